@@ -70,6 +70,9 @@ struct tzh_ctx {
     int prog_next = 0;
     // work-queue counters of persistent kernels (zero between launches)
     unsigned *work_queue = nullptr;
+    // partial results of split reductions (allocated at the first one)
+    static constexpr size_t kReduceWsBytes = (size_t)1 << 20;
+    void *reduce_ws = nullptr;
 };
 
 // Make ctx's device current for the calling thread.
@@ -79,6 +82,11 @@ int tzh_ctx_scratch(tzh_ctx *ctx, size_t bytes, void **out);
 // The context's work-queue counters (allocated and zeroed on first use;
 // the kernels that take items from them leave them at zero).
 int tzh_ctx_work_queue(tzh_ctx *ctx, unsigned **out);
+// The context's fixed workspace for the partial results of a split
+// reduction (tzh_ctx::kReduceWsBytes).  *out is null when it is not there
+// yet and cannot be allocated now (no memory, or the stream is being
+// captured): the caller then does without the split.
+int tzh_ctx_reduce_ws(tzh_ctx *ctx, void **out);
 // Stream-ordered upload of a small kernel descriptor (<= kProgSlotBytes):
 // copies `bytes` from src into the next device slot of the context's ring
 // and returns its device address, valid for kernels enqueued next on the

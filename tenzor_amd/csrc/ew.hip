@@ -42,11 +42,6 @@ using namespace tzh_ew;
 // the interpreter.
 constexpr bool kHaveJit = true;
 
-template <typename T, int V>
-struct Vec {
-    T v[V];
-};
-
 // scalar op semantics (simd.zig:107-315): ew_shared.inc
 // ------------------------------------------------------------------------
 // leaf loads
@@ -179,84 +174,82 @@ __global__ void __launch_bounds__(256) ew_chain_kernel(const EwProgram p, T *__r
     }
 }
 
-// block-wide reduction of one value per thread (256 threads)
-template <typename T>
-__device__ __forceinline__ T block_reduce(int op, T v, T *smem) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = red_apply<T>(op, v, __shfl_xor(v, o, 64));
-    const int w = threadIdx.x / 64, l = threadIdx.x % 64;
-    if (l == 0) smem[w] = v;
-    __syncthreads();
-    T r = red_ident<T>(op);
-    if (threadIdx.x == 0) {
-        for (int i = 0; i < (int)(blockDim.x / 64); i++) r = red_apply<T>(op, r, smem[i]);
-    }
-    __syncthreads();
-    return r;
-}
-
-// Reduce-all, stage 1: each block reduces a grid-stride share of the chain.
+// ------------------------------------------------------------------------
+// Reductions of a chain over [outer, rsz, inner] along rsz: the bodies are
+// reduce_rows and reduce_cols of ew_shared.inc, here over one contiguous
+// leaf and over an interpreted program (contexts that ask for the
+// interpreter); other chains run them in generated kernels (ew_jit.cpp).
+// Measured (kernel times, 16-byte loads, four vectors a thread, against one
+// thread a column or wave a row through the interpreter): mean over the
+// middle axis of f32 [256, 512, 384] 381 -> 37 us (5.4 TB/s); sum((x - y)^2)
+// over rows of [4096, 4096] 267 -> 21 us, over the middle axis of [4, 4096,
+// 4096] 13.2 ms -> 92 us (5.8 TB/s); mean of 64 rows of 100 000 830 -> 8.8.
+// The interpreter spends about 4 us on one trip of seven nodes, so it cannot
+// feed a reduction whatever its launch shape (1.1 TB/s with these shapes).
+// ------------------------------------------------------------------------
 template <typename T, int V>
-__global__ void __launch_bounds__(256) ew_reduce_all_kernel(const EwProgram p, int op,
-                                                            T *__restrict__ partials) {
-    __shared__ T smem[4];
-    T acc = red_ident<T>(op);
-    const int64_t nvec = p.numel / V;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nvec; v += stride) {
-        const Vec<T, V> r = run_program<T, V>(p, v * V);
+struct ProgSrc {
+    static constexpr int kU = 1;
+    EwProgram p;
+    __device__ __forceinline__ Batch<T, V, 1> load(const long long (&flat)[1]) const {
+        return Batch<T, V, 1>{{run_program<T, V>(p, flat[0])}};
+    }
+    __device__ __forceinline__ T load1(long long flat) const { return run_program<T, 1>(p, flat).v[0]; }
+};
+
+template <typename T, int V>
+struct LeafSrc {
+    static constexpr int kU = 4;
+    const T *p;
+    __device__ __forceinline__ Batch<T, V, kU> load(const long long (&flat)[kU]) const {
+        Batch<T, V, kU> r;
 #pragma unroll
-        for (int e = 0; e < V; e++) acc = red_apply<T>(op, acc, r.v[e]);
+        for (int u = 0; u < kU; u++) {
+            if constexpr (V * sizeof(T) == 16) {
+                const f32x4_t raw = *(const f32x4_t *)(p + flat[u]);
+                __builtin_memcpy(&r.v[u], &raw, 16);
+            } else {
+                r.v[u].v[0] = p[flat[u]];
+            }
+        }
+        return r;
     }
-    if (blockIdx.x == 0) {
-        const int64_t t = nvec * V + threadIdx.x;
-        if (t < p.numel) acc = red_apply<T>(op, acc, run_program<T, 1>(p, t).v[0]);
-    }
-    const T r = block_reduce<T>(op, acc, smem);
-    if (threadIdx.x == 0) partials[blockIdx.x] = r;
+    __device__ __forceinline__ T load1(long long flat) const { return p[flat]; }
+};
+
+template <typename T, int V, typename Src>
+__global__ void __launch_bounds__(256) ew_reduce_rows_kernel(const Src src, const RedArgs a, T *__restrict__ out) {
+    __shared__ T smem[4];
+    reduce_rows<T, V>(src, a, out, smem);
 }
 
-// Reduce-all, stage 2: one block folds the partials; mean divides by n.
+template <typename T, int V, typename Src>
+__global__ void __launch_bounds__(256) ew_reduce_cols_kernel(const Src src, const RedArgs a, T *__restrict__ out) {
+    __shared__ T smem[256 * V];
+    reduce_cols<T, V>(src, a, out, smem);
+}
+
+// Folds the parts of a split reduction, part s of output i at
+// partials[s * part_stride + i * out_stride]: blocks of 2^lx outputs by
+// 256 / 2^lx threads over the parts.  mean divides by count.
 template <typename T>
-__global__ void __launch_bounds__(256) ew_reduce_finish_kernel(const T *__restrict__ partials, int n,
-                                                               int op, int64_t count,
-                                                               T *__restrict__ out, int64_t out_numel) {
-    __shared__ T smem[4];
+__global__ void __launch_bounds__(256) ew_reduce_finish_kernel(const T *__restrict__ partials, int parts,
+                                                               int64_t part_stride, int64_t out_stride, int op,
+                                                               int64_t count, T *__restrict__ out, int64_t outs,
+                                                               int lx) {
+    __shared__ T smem[256];
+    const int x = threadIdx.x & ((1 << lx) - 1), y = threadIdx.x >> lx, ny = 256 >> lx;
+    const int64_t i = ((int64_t)blockIdx.x << lx) + x;
     T acc = red_ident<T>(op);
-    for (int i = threadIdx.x; i < n; i += blockDim.x) acc = red_apply<T>(op, acc, partials[i]);
-    T r = block_reduce<T>(op, acc, smem);
-    if (threadIdx.x == 0 && op == TZH_OP_MEAN) r = r / (T)count;
-    if (threadIdx.x == 0) smem[0] = r;
+    if (i < outs)
+        for (int s = y; s < parts; s += ny) acc = red_apply<T>(op, acc, partials[s * part_stride + i * out_stride]);
+    smem[threadIdx.x] = acc;
     __syncthreads();
-    r = smem[0];
-    for (int64_t i = threadIdx.x; i < out_numel; i += blockDim.x) out[i] = r;
-}
-
-// Reduce over the last axis (inner == 1): one wave per output row.
-template <typename T>
-__global__ void __launch_bounds__(256) ew_reduce_rows_kernel(const EwProgram p, int op, int64_t outer,
-                                                             int64_t rsz, T *__restrict__ out) {
-    const int64_t row = (int64_t)blockIdx.x * 4 + threadIdx.x / 64;
-    const int lane = threadIdx.x % 64;
-    if (row >= outer) return;
-    T acc = red_ident<T>(op);
-    for (int64_t r = lane; r < rsz; r += 64) acc = red_apply<T>(op, acc, run_program<T, 1>(p, row * rsz + r).v[0]);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) acc = red_apply<T>(op, acc, __shfl_xor(acc, o, 64));
-    if (lane == 0) out[row] = (op == TZH_OP_MEAN) ? acc / (T)rsz : acc;
-}
-
-// Reduce over a middle/leading axis: one thread per (outer, inner) column.
-template <typename T>
-__global__ void __launch_bounds__(256) ew_reduce_cols_kernel(const EwProgram p, int op, int64_t outer,
-                                                             int64_t rsz, int64_t inner,
-                                                             T *__restrict__ out) {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= outer * inner) return;
-    const int64_t o = idx / inner, i = idx % inner;
-    T acc = red_ident<T>(op);
-    for (int64_t r = 0; r < rsz; r++) acc = red_apply<T>(op, acc, run_program<T, 1>(p, (o * rsz + r) * inner + i).v[0]);
-    out[idx] = (op == TZH_OP_MEAN) ? acc / (T)rsz : acc;
+    for (int s = ny >> 1; s > 0; s >>= 1) {
+        if (y < s) smem[threadIdx.x] = acc = red_apply<T>(op, acc, smem[threadIdx.x + (s << lx)]);
+        __syncthreads();
+    }
+    if (i < outs && y == 0) out[i] = op == TZH_OP_MEAN ? acc / (T)count : acc;
 }
 
 // ------------------------------------------------------------------------
@@ -975,40 +968,115 @@ struct Planner {
         return TZH_OK;
     }
 
+    // The one leaf a program consists of when its elements lie in flat order
+    // (and, read V at a time, 16-byte aligned); else null.
+    static const void *plain_leaf(const EwProgram &p, int v) {
+        if (p.n_nodes != 1 || p.nodes[0].kind != EK_LEAF) return nullptr;
+        const EwLeaf &lf = p.leaves[p.nodes[0].arg];
+        if (lf.general || lf.div != 1 || lf.mod != INT64_MAX || (v > 1 && lf.vec != VEC_CONTIG)) return nullptr;
+        return lf.ptr;
+    }
+
+    static int log2_ceil(int64_t n) {
+        int l = 0;
+        while (((int64_t)1 << l) < n) l++;
+        return l;
+    }
+
     template <typename T, int V>
     int launch_reduce(int32_t idx, T *out) {
         const tzh_node &n = tape[idx];
         const tzh_node &c = tape[n.lhs];
-        EwProgram p;
-        const int64_t out_numel = numel_of(n.ndim, n.shape);
-        if (n.axis < 0) {
-            TZH_TRY(compile(n.lhs, p, V));
-            const int g = grid_for(p.numel / V);
-            void *partials = nullptr;
-            TZH_TRY(tzh_ctx_scratch(ctx, sizeof(T) * (size_t)g, &partials));
-            hipLaunchKernelGGL((ew_reduce_all_kernel<T, V>), dim3(g), dim3(256), 0, ctx->stream, p, n.op, (T *)partials);
-            TZH_LAUNCHED("ew_reduce_all_kernel");
-            hipLaunchKernelGGL((ew_reduce_finish_kernel<T>), dim3(1), dim3(256), 0, ctx->stream, (const T *)partials, g,
-                               n.op, p.numel, out, out_numel);
-            TZH_LAUNCHED("ew_reduce_finish_kernel");
-            return TZH_OK;
+        int64_t outer = 1, inner = 1, rsz = numel_of(c.ndim, c.shape);
+        if (n.axis >= 0) {
+            rsz = c.shape[n.axis];
+            for (int i = 0; i < n.axis; i++) outer *= c.shape[i];
+            for (int i = n.axis + 1; i < c.ndim; i++) inner *= c.shape[i];
         }
-        TZH_TRY(compile(n.lhs, p, 1));
-        int64_t outer = 1, inner = 1;
-        const int64_t rsz = c.shape[n.axis];
-        for (int i = 0; i < n.axis; i++) outer *= c.shape[i];
-        for (int i = n.axis + 1; i < c.ndim; i++) inner *= c.shape[i];
-        if (outer * inner == 0) return TZH_OK;
+        if (outer * inner == 0) {
+            EwProgram p;
+            return compile(n.lhs, p, 1);  // nothing to write; its operands are still checked
+        }
+        // V elements at a time where every row (column tile) starts on one
+        const bool vec = inner > 1 ? inner % V == 0 : rsz % V == 0 || outer == 1;
+        return vec ? reduce_with<T, V>(n, outer, rsz, inner, out) : reduce_with<T, 1>(n, outer, rsz, inner, out);
+    }
+
+    template <typename T, int V>
+    int reduce_with(const tzh_node &n, int64_t outer, int64_t rsz, int64_t inner, T *out) {
+        // A reduction reads its operands once and writes next to nothing.
+        // Both kernels aim at four blocks per CU (four waves per SIMD) and
+        // split the reduced axis where the outputs give fewer, down to parts
+        // of kMinVecs vectors per thread: the split's second launch costs
+        // about 3 us.
+        constexpr int64_t kMinVecs = 8;
+        EwProgram p;
+        TZH_TRY(compile(n.lhs, p, V));
+        const int64_t fill = (int64_t)ctx->num_cus * 4, outs = outer * inner;
+        const int64_t room = (int64_t)(tzh_ctx::kReduceWsBytes / sizeof(T)) / outs;
+        void *ws = nullptr;
+        RedArgs a{};
+        a.op = n.op, a.outer = outer, a.rsz = rsz, a.inner = inner, a.parts = 1;
+        auto split = [&](int64_t blocks, int64_t most) -> int {
+            int64_t w = (fill + blocks - 1) / blocks;
+            w = w < most ? w : most;
+            w = w < room ? w : room;
+            if (w < 2) return TZH_OK;
+            TZH_TRY(tzh_ctx_reduce_ws(ctx, &ws));  // null: none to be had now (one part)
+            if (ws) a.parts = (int)w;
+            return TZH_OK;
+        };
+        int64_t blocks;
         if (inner == 1) {
-            const int64_t blocks = (outer + 3) / 4;
-            hipLaunchKernelGGL((ew_reduce_rows_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, ctx->stream, p, n.op,
-                               outer, rsz, out);
-            TZH_LAUNCHED("ew_reduce_rows_kernel");
+            // threads per row: every lane with a vector of its own, up to a
+            // block when there are four for each
+            const int64_t nv = rsz / V;
+            a.lg = log2_ceil(nv / 4 > 16 ? nv / 4 : (nv < 16 ? nv : 16));
+            if (a.lg > 8) a.lg = 8;
+            const int64_t rows_pb = (int64_t)1 << (8 - a.lg);
+            TZH_TRY(split((outer + rows_pb - 1) / rows_pb, nv / (kMinVecs << a.lg)));
+            a.part_len = (nv + a.parts - 1) / a.parts;
+            blocks = (outer * a.parts + rows_pb - 1) / rows_pb;
         } else {
-            const int64_t blocks = (outer * inner + 255) / 256;
-            hipLaunchKernelGGL((ew_reduce_cols_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, ctx->stream, p, n.op,
-                               outer, rsz, inner, out);
-            TZH_LAUNCHED("ew_reduce_cols_kernel");
+            // column vectors per block: 64 (whole waves along a row) unless a
+            // narrower tile leaves fewer lanes idle
+            const int64_t ncv = (inner + V - 1) / V;
+            a.lg = 6;
+            while (a.lg > 4 && (((ncv - 1) >> a.lg) + 1) << a.lg > ncv + ncv / 8) a.lg--;
+            if (ncv < 16) a.lg = log2_ceil(ncv);
+            a.tiles = ((ncv - 1) >> a.lg) + 1;
+            TZH_TRY(split(a.tiles * outer, rsz / (kMinVecs * (256 >> a.lg))));
+            a.part_len = (rsz + a.parts - 1) / a.parts;
+            blocks = a.tiles * outer * a.parts;
+        }
+        if (blocks > INT32_MAX) return tzh_fail(TZH_ERR_TOO_LARGE, "reduction to %lld elements", (long long)outs);
+        a.finish = a.parts == 1;
+        T *const dst = a.finish ? out : (T *)ws;
+        const dim3 grid((unsigned)blocks);
+        if (const void *leaf = plain_leaf(p, V)) {
+            const LeafSrc<T, V> src{(const T *)leaf};
+            if (inner == 1)
+                hipLaunchKernelGGL((ew_reduce_rows_kernel<T, V, LeafSrc<T, V>>), grid, dim3(256), 0, ctx->stream, src, a, dst);
+            else
+                hipLaunchKernelGGL((ew_reduce_cols_kernel<T, V, LeafSrc<T, V>>), grid, dim3(256), 0, ctx->stream, src, a, dst);
+        } else if (kHaveJit && !ctx->ew_interpreter) {
+            TZH_TRY(jit_reduce_launch(ctx, p, a, sizeof(T) == 8, V, (int)blocks, dst));
+        } else {
+            const ProgSrc<T, V> src{p};
+            if (inner == 1)
+                hipLaunchKernelGGL((ew_reduce_rows_kernel<T, V, ProgSrc<T, V>>), grid, dim3(256), 0, ctx->stream, src, a, dst);
+            else
+                hipLaunchKernelGGL((ew_reduce_cols_kernel<T, V, ProgSrc<T, V>>), grid, dim3(256), 0, ctx->stream, src, a, dst);
+        }
+        TZH_LAUNCHED("ew_reduce kernel");
+        const int parts = a.parts;
+        if (parts > 1) {
+            // [outer][parts], a block per output, or [parts][outer * inner]
+            const int lx = inner == 1 ? 0 : 4;
+            hipLaunchKernelGGL((ew_reduce_finish_kernel<T>), dim3((unsigned)((outs + (1 << lx) - 1) >> lx)), dim3(256),
+                               0, ctx->stream, (const T *)ws, parts, inner == 1 ? 1 : outs, inner == 1 ? parts : 1, n.op,
+                               rsz, out, outs, lx);
+            TZH_LAUNCHED("ew_reduce_finish_kernel");
         }
         return TZH_OK;
     }

@@ -1,4 +1,4 @@
-// Generated single-pass chain kernels (K1 fast path).
+// Generated single-pass chain and reduction kernels (K1 fast path).
 //
 // The reference fuses an elementwise chain at compile time into one loop
 // (codegen.zig:15-205 FusedElementwiseKernel: the ops of the chain applied
@@ -44,7 +44,7 @@ const char kSharedSrc[] =
     X(TZH_OP_NEG) X(TZH_OP_ABS) X(TZH_OP_EXP) X(TZH_OP_LOG) X(TZH_OP_SQRT) X(TZH_OP_RSQRT) X(TZH_OP_SIN)   \
     X(TZH_OP_COS) X(TZH_OP_TANH) X(TZH_OP_SIGMOID) X(TZH_OP_RELU) X(TZH_OP_GELU) X(TZH_OP_SILU)           \
     X(TZH_OP_SOFTPLUS) X(TZH_OP_FLOOR) X(TZH_OP_CEIL) X(TZH_OP_ROUND) X(TZH_OP_ADD) X(TZH_OP_SUB)         \
-    X(TZH_OP_MUL) X(TZH_OP_DIV) X(TZH_OP_POW) X(TZH_OP_MAX) X(TZH_OP_MIN) X(TZH_OP_PROD)                  \
+    X(TZH_OP_MUL) X(TZH_OP_DIV) X(TZH_OP_POW) X(TZH_OP_MAX) X(TZH_OP_MIN) X(TZH_OP_SUM) X(TZH_OP_MEAN) X(TZH_OP_PROD)                  \
     X(TZH_OP_REDUCE_MAX) X(TZH_OP_REDUCE_MIN)
 
 std::string prelude() {
@@ -236,19 +236,93 @@ std::string chain_source(const EwProgram &p, bool f64, int V) {
     return s;
 }
 
+// Reduction kernel (reduce_rows or reduce_cols of ew_shared.inc) whose
+// operand is the chain: Src::load reads every leaf of kU vectors before any
+// arithmetic.
+std::string reduce_source(const EwProgram &p, bool cols, bool f64, int V) {
+    constexpr int U = 4;
+    const std::string T = f64 ? "double" : "float", VS = std::to_string(V), US = std::to_string(U);
+    const bool vec16 = V * (f64 ? 8 : 4) == 16;
+    std::string s = prelude();
+    for (int j = 0; j < p.n_leaves; j++) s += offset_fn(p, j);
+    s += "struct Src {\n    static constexpr int kU = " + US + ";\n    const EwProgram &p;\n";
+    s += "    __device__ __forceinline__ Batch<" + T + ", " + VS + ", kU> load(const long long (&flat)[kU]) const {\n";
+    s += "        Batch<" + T + ", " + VS + ", kU> r;\n";
+    for (int u = 0; u < U; u++) s += loads(p, T.c_str(), V, vec16, "_" + std::to_string(u), "flat[" + std::to_string(u) + "]");
+    for (int u = 0; u < U; u++) {
+        const std::string S = "_" + std::to_string(u);
+        s += "        " + T + " r" + S + "[" + VS + "];\n" + compute(p, T.c_str(), V, S);
+        for (int e = 0; e < V; e++) {
+            const std::string E = std::to_string(e);
+            s += "        r.v[" + std::to_string(u) + "].v[" + E + "] = r" + S + "[" + E + "];\n";
+        }
+    }
+    s += "        return r;\n    }\n";
+    s += "    __device__ __forceinline__ " + T + " load1(long long flat) const {\n";
+    s += loads(p, T.c_str(), 1, false, "", "flat");
+    s += "        " + T + " r[1];\n" + compute(p, T.c_str(), 1, "") + "        return r[0];\n    }\n};\n";
+    s += "extern \"C\" __global__ void __launch_bounds__(256) tzh_reduce(const EwProgram p, const RedArgs a, " + T +
+         " *__restrict__ out) {\n    __shared__ " + T + " smem[" + (cols ? "256 * " + VS : std::string("4")) + "];\n" +
+         "    reduce_" + (cols ? "cols" : "rows") + "<" + T + ", " + VS + ">(Src{p}, a, out, smem);\n}\n";
+    return s;
+}
+
+enum Form : char { kChainForm, kRowsForm, kColsForm };
+
+std::string source_of(const EwProgram &p, Form form, bool f64, int V) {
+    return form == kChainForm ? chain_source(p, f64, V) : reduce_source(p, form == kColsForm, f64, V);
+}
+
+// What the generated text depends on, in a few hundred bytes: kernels are
+// looked up by it, so that a call whose kernel exists builds no text (writing
+// and hashing the text took 10 us of a 24 us call).
+std::string key_of(int device, const EwProgram &p, Form form, bool f64, int V) {
+    std::string k;
+    k.reserve(16 + 8 * (size_t)p.n_nodes + 16 * (size_t)p.n_leaves);
+    auto put = [&](long long v, int bytes) {
+        for (int i = 0; i < bytes; i++) k.push_back((char)((unsigned long long)v >> (8 * i)));
+    };
+    put(device, 4);
+    put(form, 1);
+    put(f64, 1);
+    put(V, 1);
+    put(p.small, 1);
+    put(p.ndim, 1);
+    put(p.n_nodes, 1);
+    put(p.n_leaves, 1);
+    for (int i = 0; i < p.n_nodes; i++) {
+        const EwNode &nd = p.nodes[i];
+        put(nd.kind, 1);
+        put(nd.op, 2);
+        put(nd.slot, 1);
+        put(nd.arg, 1);
+    }
+    for (int j = 0; j < p.n_leaves; j++) {
+        const EwLeaf &lf = p.leaves[j];
+        put(lf.general, 1);
+        put(lf.vec, 1);
+        put(lf.div != 1, 1);
+        put(lf.mod <= (long long)0xffffffff, 1);
+        int strided = 0;
+        for (int d = 0; d < p.ndim; d++) strided |= (lf.strides[d] != 0) << d;
+        put(strided, 1);
+    }
+    return k;
+}
+
 #ifdef TZH_EMULATION
 // CPU emulation build (tests/cpu_emu; test infrastructure only): the same
 // generated text is compiled as C++ against the emulated runtime header,
 // with AddressSanitizer, into a shared object linked to the emulation
 // library, and its kernel is run on the emulator's fibers.  The compiler
 // and header directory are fixed when the emulation library is built.
-using EmuLaunch = void (*)(unsigned grid, const void *p, void *out);
+using EmuLaunch = void (*)(unsigned grid, const void *p, const void *a, void *out);
 
 std::mutex g_mu;
-std::unordered_map<std::string, EmuLaunch> g_cache;  // key: source
+std::unordered_map<std::string, EmuLaunch> g_cache;  // by key_of
 std::string g_dir;
 
-int emu_compile(const std::string &src, bool f64, EmuLaunch *out) {
+int emu_compile(const std::string &src, bool f64, bool reduce, EmuLaunch *out) {
     if (g_dir.empty()) {
         char tmpl[] = "/tmp/tzh_emu_jit_XXXXXX";
         if (!mkdtemp(tmpl)) return tzh_fail(TZH_ERR_DEVICE, "emulated chain kernel: mkdtemp failed");
@@ -260,9 +334,11 @@ int emu_compile(const std::string &src, bool f64, EmuLaunch *out) {
     const std::string stem = g_dir + "/k" + std::to_string(g_cache.size());
     const char *T = f64 ? "double" : "float";
     std::string text = "#include \"hip/hip_runtime.h\"\n" + src;
-    text += "extern \"C\" void tzh_chain_emu_launch(unsigned grid, const void *p, void *out) {\n"
-            "    emu::launch_kernel(\"tzh_chain (generated)\", tzh_chain, dim3(grid), dim3(256),\n"
-            "                       *(const EwProgram *)p, (" + std::string(T) + " *)out);\n}\n";
+    const std::string kernel = reduce ? "tzh_reduce" : "tzh_chain";
+    text += "extern \"C\" void tzh_chain_emu_launch(unsigned grid, const void *p, const void *a, void *out) {\n"
+            "    emu::launch_kernel(\"" + kernel + " (generated)\", " + kernel + ", dim3(grid), dim3(256),\n"
+            "                       *(const EwProgram *)p, " + (reduce ? "*(const RedArgs *)a, " : "") + "(" +
+            std::string(T) + " *)out);\n}\n";
     FILE *f = std::fopen((stem + ".cpp").c_str(), "w");
     if (!f) return tzh_fail(TZH_ERR_DEVICE, "emulated chain kernel: cannot write %s.cpp", stem.c_str());
     std::fwrite(text.data(), 1, text.size(), f);
@@ -281,22 +357,33 @@ int emu_compile(const std::string &src, bool f64, EmuLaunch *out) {
 
 }  // namespace
 
-int jit_chain_launch(tzh_ctx *ctx, const EwProgram &p, bool f64, int V, int grid, void *out) {
-    (void)ctx;
-    const std::string src = chain_source(p, f64, V);
+namespace {
+
+int emu_launch(Form form, const EwProgram &p, const RedArgs *a, bool f64, int V, int grid, void *out) {
     EmuLaunch fn = nullptr;
     {
+        const std::string key = key_of(0, p, form, f64, V);
         std::lock_guard<std::mutex> lock(g_mu);
-        auto it = g_cache.find(src);
+        auto it = g_cache.find(key);
         if (it == g_cache.end()) {
-            TZH_TRY(emu_compile(src, f64, &fn));
-            g_cache.emplace(src, fn);
+            TZH_TRY(emu_compile(source_of(p, form, f64, V), f64, a != nullptr, &fn));
+            g_cache.emplace(key, fn);
         } else {
             fn = it->second;
         }
     }
-    fn((unsigned)grid, &p, out);
+    fn((unsigned)grid, &p, a, out);
     return TZH_OK;
+}
+
+}  // namespace
+
+int jit_chain_launch(tzh_ctx *, const EwProgram &p, bool f64, int V, int grid, void *out) {
+    return emu_launch(kChainForm, p, nullptr, f64, V, grid, out);
+}
+
+int jit_reduce_launch(tzh_ctx *, const EwProgram &p, const RedArgs &a, bool f64, int V, int grid, void *out) {
+    return emu_launch(a.inner > 1 ? kColsForm : kRowsForm, p, &a, f64, V, grid, out);
 }
 
 #else
@@ -306,9 +393,9 @@ struct Compiled {
 };
 
 std::mutex g_mu;
-std::unordered_map<std::string, Compiled> g_cache;  // key: device id + source
+std::unordered_map<std::string, Compiled> g_cache;  // by key_of
 
-int compile(int device, const std::string &src, Compiled *out) {
+int compile(int device, const std::string &src, const char *kernel, Compiled *out) {
     hipDeviceProp_t prop;
     TZH_HIP(hipGetDeviceProperties(&prop, device));
     std::string arch = prop.gcnArchName;
@@ -337,29 +424,42 @@ int compile(int device, const std::string &src, Compiled *out) {
     hiprtcGetCode(prog, code.data());
     hiprtcDestroyProgram(&prog);
     TZH_HIP(hipModuleLoadData(&out->module, code.data()));
-    TZH_HIP(hipModuleGetFunction(&out->fn, out->module, "tzh_chain"));
+    TZH_HIP(hipModuleGetFunction(&out->fn, out->module, kernel));
+    return TZH_OK;
+}
+
+// The kernel of a program in one form, compiled at its first use on the device.
+int lookup(tzh_ctx *ctx, const EwProgram &p, Form form, bool f64, int V, hipFunction_t *fn) {
+    const std::string key = key_of(ctx->device, p, form, f64, V);
+    std::lock_guard<std::mutex> lock(g_mu);
+    auto it = g_cache.find(key);
+    if (it == g_cache.end()) {
+        Compiled k{};
+        TZH_TRY(compile(ctx->device, source_of(p, form, f64, V), form == kChainForm ? "tzh_chain" : "tzh_reduce", &k));
+        it = g_cache.emplace(key, k).first;
+    }
+    *fn = it->second.fn;
     return TZH_OK;
 }
 
 }  // namespace
 
 int jit_chain_launch(tzh_ctx *ctx, const EwProgram &p, bool f64, int V, int grid, void *out) {
-    const std::string src = chain_source(p, f64, V);
-    const std::string key = std::to_string(ctx->device) + "\n" + src;
-    Compiled k{};
-    {
-        std::lock_guard<std::mutex> lock(g_mu);
-        auto it = g_cache.find(key);
-        if (it == g_cache.end()) {
-            TZH_TRY(compile(ctx->device, src, &k));
-            g_cache.emplace(key, k);
-        } else {
-            k = it->second;
-        }
-    }
+    hipFunction_t fn;
+    TZH_TRY(lookup(ctx, p, kChainForm, f64, V, &fn));
     EwProgram arg = p;
     void *args[] = {&arg, &out};
-    TZH_HIP(hipModuleLaunchKernel(k.fn, (unsigned)grid, 1, 1, 256, 1, 1, 0, ctx->stream, args, nullptr));
+    TZH_HIP(hipModuleLaunchKernel(fn, (unsigned)grid, 1, 1, 256, 1, 1, 0, ctx->stream, args, nullptr));
+    return TZH_OK;
+}
+
+int jit_reduce_launch(tzh_ctx *ctx, const EwProgram &p, const RedArgs &a, bool f64, int V, int grid, void *out) {
+    hipFunction_t fn;
+    TZH_TRY(lookup(ctx, p, a.inner > 1 ? kColsForm : kRowsForm, f64, V, &fn));
+    EwProgram arg = p;
+    RedArgs red = a;
+    void *args[] = {&arg, &red, &out};
+    TZH_HIP(hipModuleLaunchKernel(fn, (unsigned)grid, 1, 1, 256, 1, 1, 0, ctx->stream, args, nullptr));
     return TZH_OK;
 }
 

@@ -43,4 +43,8 @@ inline bool unary_ok(int op) {
 // compiled on first use of a program shape and cached per device.
 int jit_chain_launch(tzh_ctx *ctx, const EwProgram &p, bool f64, int V, int grid, void *out);
 
+// The same for a reduction of program p: reduce_rows (a.inner == 1) or
+// reduce_cols over the generated operand, `grid` blocks of 256 threads.
+int jit_reduce_launch(tzh_ctx *ctx, const EwProgram &p, const RedArgs &a, bool f64, int V, int grid, void *out);
+
 }  // namespace tzh_ew

@@ -108,6 +108,23 @@ int tzh_ctx_work_queue(tzh_ctx *ctx, unsigned **out) {
     return TZH_OK;
 }
 
+int tzh_ctx_reduce_ws(tzh_ctx *ctx, void **out) {
+    *out = ctx->reduce_ws;
+    if (*out) return TZH_OK;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) {  // e.g. the default stream during another's capture
+        (void)hipGetLastError();
+        return TZH_OK;
+    }
+    if (cap != hipStreamCaptureStatusNone) return TZH_OK;
+    if (hipMalloc(&ctx->reduce_ws, tzh_ctx::kReduceWsBytes) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->reduce_ws = nullptr;
+    }
+    *out = ctx->reduce_ws;
+    return TZH_OK;
+}
+
 int tzh_ctx_upload_program(tzh_ctx *ctx, const void *src, size_t bytes, const void **dev_out) {
     if (bytes > tzh_ctx::kProgSlotBytes) return tzh_fail(TZH_ERR_INVALID_ARGS, "internal: program of %zu bytes", bytes);
     if (!ctx->prog_dev) {
@@ -149,6 +166,7 @@ extern "C" int tzh_destroy(tzh_ctx *ctx) {
     if (ctx->prog_host) hipHostFree(ctx->prog_host);
     if (ctx->scratch) hipFree(ctx->scratch);
     if (ctx->work_queue) hipFree(ctx->work_queue);
+    if (ctx->reduce_ws) hipFree(ctx->reduce_ws);
     if (ctx->own_stream) hipStreamDestroy(ctx->stream);
     delete ctx;
     return TZH_OK;

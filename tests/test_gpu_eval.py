@@ -215,6 +215,44 @@ def test_reduce_vs_oracle(ctx, op, axes, keep):
     np.testing.assert_allclose(out, ref, rtol=2e-5 if op != "prod" else 2e-4)
 
 
+@pytest.mark.parametrize("chain", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("shape,axis", [
+    ((5, 1), 1), ((1, 3), 1), ((300, 7), 1), ((9, 64), 1), ((3, 255), 1), ((3, 260), 1), ((2, 1028), 1),
+    ((1, 70001), 1), ((2, 9000), 1), ((70003,), None), ((3,), None), ((4, 5, 6), None),
+    ((1, 2), 0), ((2, 3, 2), 1), ((3, 40, 5), 1), ((33, 16), 0), ((7, 68), 0), ((2, 9, 260), 1), ((1500, 12), 0),
+    ((1, 700, 65), 1),
+])
+def test_reduce_launch_shapes(ctx, shape, axis, dtype, chain):
+    """The edges of the reduction kernels' launch rules: fewer elements than
+    lanes, one group size to the next, rows and columns that are not whole
+    vectors, tiles partly past the last column, splits along the reduced axis
+    with a short last part; one leaf (aligned and not) and a chain.  Each sum
+    of n terms of either side is within n rounding errors of its terms'
+    magnitude; maxima are exact."""
+    np_dt = np.float32 if dtype == torch.float32 else np.float64
+    rng = np.random.default_rng(11)
+    n = int(np.prod(shape))
+    flat = rng.standard_normal(n + 1).astype(np_dt)
+    dev = torch.from_numpy(flat).to(DEV)
+    eps = float(np.finfo(np_dt).eps)
+    axes = () if axis is None else (axis,)
+    for off in (0, 1):  # off 1: the leaf is not 16-byte aligned
+        x = flat[off:off + n].reshape(shape)
+        leaf = Tensor(dev[off:off + n].view(shape))
+        e = leaf.sub(0.25).mul(leaf) if chain else leaf
+        v = ((x - np_dt(0.25)) * x if chain else x).astype(np.float64)
+        terms = n if axis is None else shape[axis]
+        mag = np.abs(v).sum(axis=axis)
+        for op, ref in (("sum", v.sum(axis=axis)), ("mean", v.mean(axis=axis)), ("reduce_max", v.max(axis=axis))):
+            got = eval(ReduceExpr(op, e, axes), ctx).cpu().numpy().astype(np.float64)
+            # the chain's own two roundings, then at most one per addition (and one for the division)
+            bound = 2 * eps * (np.abs(ref) if op == "reduce_max" else (terms + 3) * mag / (terms if op == "mean" else 1))
+            if op == "reduce_max" and not chain:
+                bound = 0
+            assert (np.abs(got - ref) <= bound + (0 if not chain else 2 * eps)).all(), (op, off)
+
+
 def test_reduce_feeds_chain(ctx):
     rng = np.random.default_rng(6)
     x = rng.standard_normal((40, 300)).astype(np.float32)
