@@ -469,7 +469,7 @@ int32_t model_act(const tzh_model *m) {
 
 // y[T, n] = ops(x[T, k] W^T) + C for an f32-weight linear (W [n, k]), ops =
 // bias add then `act_op` (or the bias add alone when act_op < 0).
-int linear_f32w(hipStream_t st, const float *x, const DevLinear &l, float *y, int64_t T, int64_t k, int64_t n,
+int linear_f32w(hipStream_t st, int num_cus, const float *x, const DevLinear &l, float *y, int64_t T, int64_t k, int64_t n,
                 int act_op, const float *residual) {
     tzh_gemm_desc d;
     d.m = T, d.n = n, d.k = k, d.lda = k, d.ldb = k, d.ldy = n;
@@ -478,7 +478,8 @@ int linear_f32w(hipStream_t st, const float *x, const DevLinear &l, float *y, in
     d.n_ops = 1;
     if (act_op >= 0) d.ops[d.n_ops++] = act_op;
     if (residual) d.c = residual, d.beta = 1.0, d.c_rs = n, d.c_cs = 1;
-    return tzh_gemm_fp_launch(st, TZH_F32, false, true, x, l.w, y, d);
+    d.split_k = false;  // a row's sums in the same order whatever the batch
+    return tzh_gemm_fp_launch(st, num_cus, TZH_F32, false, true, x, l.w, y, d);
 }
 
 int layernorm_rows(hipStream_t st, const float *x, const float *g, const float *b, float *y, int64_t rows, int n,
@@ -510,12 +511,12 @@ int ffn_part(tzh_model *m, const DevLayer &d, hipStream_t st, int32_t act, bool 
                                     nullptr, m->mlp_tail, m->mlp_tail_bytes);
     if (part == 1) {
         if (d.ffn1.fmt == TZH_WF_F32)
-            return linear_f32w(st, (const float *)x, d.ffn1, (float *)m->inter, T, H, 1536, TZH_OP_GELU, nullptr);
+            return linear_f32w(st, cus, (const float *)x, d.ffn1, (float *)m->inter, T, H, 1536, TZH_OP_GELU, nullptr);
         return tzh_linear_codes_launch(st, cus, x, act, d.ffn1.w, d.ffn1.fmt, d.ffn1.s, d.ffn1.b, m->inter, act, T, H,
                                        1536, 1536, TZH_EPI_BIAS_GELU, nullptr, nullptr, nullptr, 0.0f, nullptr, 0, rs);
     }
     if (d.ffn2.fmt == TZH_WF_F32) {
-        TZH_TRY(linear_f32w(st, (const float *)m->inter, d.ffn2, (float *)m->attn, T, 1536, H, -1, (const float *)x));
+        TZH_TRY(linear_f32w(st, cus, (const float *)m->inter, d.ffn2, (float *)m->attn, T, 1536, H, -1, (const float *)x));
         return layernorm_rows(st, (const float *)m->attn, d.ln2_g, d.ln2_b, (float *)y, T, H, eps);
     }
     return tzh_linear_codes_launch(st, cus, m->inter, act, d.ffn2.w, d.ffn2.fmt, d.ffn2.s, d.ffn2.b, y, act, T, 1536, H,
@@ -1016,7 +1017,7 @@ int run_forward(tzh_model *m, float *outputs, float *hidden_out, const uint32_t 
         // inside the split's range (set_range)
         const bool rs = m->row_scaled && act == TZH_F32;
         TZH_TRY(stage("qkv", [&]() {
-            if (d.qkv.fmt == TZH_WF_F32) return linear_f32w(st, hf, d.qkv, (float *)m->qkv, T, H, 3 * H, -1, nullptr);
+            if (d.qkv.fmt == TZH_WF_F32) return linear_f32w(st, cus, hf, d.qkv, (float *)m->qkv, T, H, 3 * H, -1, nullptr);
             // int8 QKV of the f32 forward on the fused kernel's QKV mode
             // (X in registers, the weights streamed through LDS)
             if (m->fuse_ffn && d.qkvp && act == TZH_F32 && !rs)
@@ -1044,7 +1045,7 @@ int run_forward(tzh_model *m, float *outputs, float *hidden_out, const uint32_t 
         }
         TZH_TRY(stage("attn_out_ln", [&]() {
             if (d.o.fmt == TZH_WF_F32) {
-                TZH_TRY(linear_f32w(st, (const float *)m->attn, d.o, (float *)m->inter, T, H, H, -1, hf));
+                TZH_TRY(linear_f32w(st, cus, (const float *)m->attn, d.o, (float *)m->inter, T, H, H, -1, hf));
                 return layernorm_rows(st, (const float *)m->inter, d.ln1_g, d.ln1_b, h1f, T, H, eps);
             }
             return tzh_linear_codes_launch(st, cus, m->attn, act, d.o.w, d.o.fmt, d.o.s, d.o.b, m->h1, act, T, H, H,

@@ -112,10 +112,13 @@ struct tzh_gemm_desc {
     const void *bias = nullptr;
     int32_t n_ops = 0;
     int32_t ops[4] = {};
+    // allow tiles that split k over a block's waves: their sums run in
+    // another order than the other tiles', which all share one
+    bool split_k = true;
 };
 // a_trans: A stored [k][m]; b_trans: B stored [n][k].
-int tzh_gemm_fp_launch(hipStream_t st, int32_t dtype, bool a_trans, bool b_trans, const void *a, const void *b,
-                       void *y, const tzh_gemm_desc &d);
+int tzh_gemm_fp_launch(hipStream_t st, int num_cus, int32_t dtype, bool a_trans, bool b_trans, const void *a,
+                       const void *b, void *y, const tzh_gemm_desc &d);
 
 // Host tokenizer (tokenizer.cpp) for the embedding entry points.
 size_t tzh_tokenize(const tzh_tokenizer *tok, const uint8_t *text, size_t len, uint32_t *out, size_t cap);

@@ -1259,7 +1259,7 @@ struct Planner {
         d.bias = bias;
         d.n_ops = n_ops;
         for (int o = 0; o < n_ops; o++) d.ops[o] = ops[o];
-        return tzh_gemm_fp_launch(ctx->stream, dtype, false, false, adat, bdat, out, d);
+        return tzh_gemm_fp_launch(ctx->stream, ctx->num_cus, dtype, false, false, adat, bdat, out, d);
     }
 
     // A row vector over the last axis of a result of rank nd: a leaf whose

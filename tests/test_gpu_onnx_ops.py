@@ -60,6 +60,27 @@ def test_gemm_vs_oracle(ctx, ta, tb, m, n, k, cshape):
     assert (np.abs(y - ref) <= bound(A, B, 0.75, ta, tb, ref) + 2.0 ** -23 * 1.5 * (0 if Cm is None else np.abs(Cm).max())).all()
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("m,n,k", [(4101, 4100, 17),   # 128 x 128 tiles on 256 CUs
+                                   (4090, 1530, 33),   # 64 x 128
+                                   (1000, 1003, 65), (65, 6400, 1),   # 64 x 64
+                                   (31, 33, 129), (1, 300, 257), (513, 40, 128)])  # 32 x 32
+def test_gemm_tile_shapes(ctx, ta, tb, m, n, k):
+    """Each tile shape at sizes that leave partial tiles and a short last k
+    stage, for every storage order, against a float64 product; bound: each
+    of the k products and sums rounds once."""
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    A = torch.randn((k, m) if ta else (m, k), device="cuda", generator=g)
+    B = torch.randn((n, k) if tb else (k, n), device="cuda", generator=g)
+    Y = torch.full((m, n), float("nan"), device="cuda")
+    check(lib().tzh_gemm_f32(ctx.handle, ta, tb, m, n, k, 1.0, A.data_ptr(), A.shape[1], B.data_ptr(), B.shape[1], 0.0,
+                             None, 0, 0, Y.data_ptr()))
+    a64 = (A.t() if ta else A).double().contiguous()
+    b64 = (B.t() if tb else B).double().contiguous()
+    ref, mag = a64 @ b64, a64.abs() @ b64.abs()
+    assert bool(((Y.double() - ref).abs() <= mag * (k + 2) * 2.0 ** -24 + 2.0 ** -23 * ref.abs()).all())
+
+
 def test_gemm_row_pitch_and_unaligned(ctx):
     """Row pitches larger than the row (lda > k) and operands off 16-byte
     boundaries (scalar loads)."""
