@@ -184,9 +184,10 @@ int tzh_eval_into(tzh_ctx *ctx, const tzh_node *tape, int32_t n_nodes,
  * to 2^-22 relative for every value within 2^17 of its row's largest), the
  * sums run in f32 and are multiplied by 2^-e (exact) before the scale and
  * bias.  Rows holding inf or NaN give NaN where the reference gives inf or
- * NaN.  The int8 codes are rewritten into the kernel's tiled format in the
- * context scratch on every call (with the row exponents, and a copy of a
- * with zero columns when k % 64 != 0). */
+ * NaN.  With few rows the codes are read where they are; otherwise they are
+ * rewritten into the kernel's tiled format in the context scratch on every
+ * call (with the row exponents, and a copy of a with zero columns when
+ * k % 64 != 0). */
 int tzh_matmul_w8a32(tzh_ctx *ctx, const float *a, const int8_t *wq, const uint16_t *scale,
                      const float *bias, float *c, int64_t m, int64_t k, int64_t n);
 

@@ -3,7 +3,9 @@
 // calls Arctic makes after it (GELU, arctic.zig:771-776; residual +
 // LayerNorm, arctic.zig:716-746, 779-809).
 //
-// Every shape runs on the pipelined MFMA kernel of gemm_pipe.hip.  Per call
+// Few rows run on linear_small_kernel (linear_small.hip), which reads the
+// codes and rows as they are.  Other shapes run on the pipelined MFMA kernel
+// of gemm_pipe.hip.  Per call
 // the int8 codes [n, k] are rewritten into its stage-tiled format, padded to
 // n_pad (a multiple of 384) rows and k_pad (a multiple of 64) columns with
 // code 0; when k is not a multiple of 64 the activation rows are copied with
@@ -33,6 +35,13 @@ int tzh_linear_codes_launch(hipStream_t st, int num_cus, const void *x, int32_t 
                             int64_t m, int64_t k, int64_t n, int64_t n_valid, int32_t epilogue, const void *res,
                             const float *gamma, const float *beta, float eps, float *ln_ws, int64_t ln_ws_rows,
                             bool row_scale);
+
+bool tzh_linear_small_wins(int64_t m, int64_t k, int64_t n, bool f32, bool ln);
+int tzh_linear_small_launch(hipStream_t st, int num_cus, const void *x, int32_t x_dtype, const int8_t *q,
+                            const uint16_t *scale, const float *bias, void *c, int32_t c_dtype, int64_t m, int64_t k,
+                            int64_t n, int32_t epilogue, const void *res, float *pre_ln);
+int tzh_ln_rows_launch(hipStream_t st, const float *rows, int64_t m, const float *gamma, const float *beta, float eps,
+                       void *out, int32_t dtype);
 
 namespace {
 
@@ -145,6 +154,19 @@ int linear(tzh_ctx *ctx, const void *a, int32_t a_dtype, const int8_t *wq, const
     if (((uintptr_t)c & 3) || (ln && !al16(c)))
         return tzh_fail(TZH_ERR_INVALID_ARGS, "c is not aligned to its element (16 bytes with the LayerNorm epilogue)");
     const Workspace wsz = workspace_of(ctx, a, a_dtype, m, k, n, ln);
+    if (tzh_linear_small_wins(m, k, n, a_dtype == TZH_F32, ln) && (!ln || m <= wsz.ws_rows)) {
+        // few rows: the codes and rows are read as they are, and the
+        // LayerNorm epilogue's rows wait in the workspace
+        float *rows = nullptr;
+        if (ln) {
+            void *sp = scratch_ptr;
+            if (!sp) TZH_TRY(tzh_ctx_scratch(ctx, wsz.total(), &sp));
+            rows = (float *)sp;
+        }
+        TZH_TRY(tzh_linear_small_launch(ctx->stream, ctx->num_cus, a, a_dtype, wq, scale, bias, c, c_dtype, m, k, n,
+                                        epilogue, residual, rows));
+        return ln ? tzh_ln_rows_launch(ctx->stream, rows, m, gamma, beta, eps, c, c_dtype) : TZH_OK;
+    }
     const bool pad_a = wsz.a > 0;
     const size_t codes_bytes = wsz.codes, a_bytes = wsz.a;
     const int64_t ws_rows = wsz.ws_rows;

@@ -123,27 +123,6 @@ __device__ __forceinline__ void store_frag_f32(char *ws, const f32x16_t &v, floa
     wave_lds_order();
 }
 
-// Eight biased int8 weight codes (u = q + 128, little-endian in d0, d1) ->
-// f16 q, exactly: v_perm_b32 makes each code the low mantissa byte of an f16
-// with exponent 10 (bits 0x64uu = 1024 + u), and a packed f16 subtraction of
-// 1152 = 1024 + 128 leaves q; every value is an integer below 2048, so
-// nothing rounds.
-__device__ __forceinline__ half8_t codes_to_f16(uint32_t d0, uint32_t d1) {
-    const half2_t off = {(_Float16)1152.0f, (_Float16)1152.0f};
-    half8_t r;
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const uint32_t d = i ? d1 : d0;
-        const half2_t lo = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, d, 0x04010400u)) - off;
-        const half2_t hi = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, d, 0x04030402u)) - off;
-        r[4 * i + 0] = lo[0];
-        r[4 * i + 1] = lo[1];
-        r[4 * i + 2] = hi[0];
-        r[4 * i + 3] = hi[1];
-    }
-    return r;
-}
-
 // Tile of rows x ROW_BYTES (k contiguous) as laid out in LDS.
 template <int ROW_BYTES_>
 struct TileFmt {
@@ -1070,6 +1049,20 @@ __global__ void tile_codes_w8_kernel(const int8_t *__restrict__ q, uint8_t *__re
 bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
+
+// out [m, 384] (F32 or F16) = LayerNorm of m f32 rows, statistics in the
+// order of the GEMM's LayerNorm epilogue.
+int tzh_ln_rows_launch(hipStream_t st, const float *rows, int64_t m, const float *gamma, const float *beta, float eps,
+                       void *out, int32_t dtype) {
+    const dim3 grid((unsigned)((m + 31) / 32));
+    if (dtype == TZH_F32)
+        hipLaunchKernelGGL(ln_rows_kernel<float>, grid, dim3(256), 0, st, rows, (int)m, gamma, beta, eps, (float *)out);
+    else
+        hipLaunchKernelGGL(ln_rows_kernel<_Float16>, grid, dim3(256), 0, st, rows, (int)m, gamma, beta, eps,
+                           (_Float16 *)out);
+    TZH_LAUNCHED("ln_rows_kernel");
+    return TZH_OK;
+}
 
 // int8 codes [n, k] -> the TZH_WF_W8T layout of the padded shape n_pad x
 // k_pad (multiples of 384 and 64, at least n and k).

@@ -1,0 +1,401 @@
+// The int8-weight linear for few rows:
+//
+//   C[t, n] = epi( (sum_k X[t,k] * q[n,k]) * f32(scale[n]) + bias[n] )
+//
+// the sums and arithmetic of gemm_pipe.hip (matmul_w8a32.zig:14-57: f32
+// activations as exact f16 halves hi + lo, codes exact in f16, f32 sums;
+// f16 activations as they are), for problems whose 128 x 384 tiles would
+// leave most of the chip idle and walk k as one long chain of stages.
+//
+// Bound by latency, so the design shortens the chain:
+//   - Blocks of 16 or 32 rows by 64 outputs (four waves, 16 outputs each) or
+//     16 rows by 16 outputs (the four waves share k): enough blocks for the
+//     chip at any size this kernel is used for.
+//   - A block holds its rows' k range (chunks of 512 or 1024) in LDS, split
+//     into f16 halves once.  Every load of a chunk - the wave's codes
+//     straight into registers, the rows - is issued before the first wait;
+//     nothing is staged in rounds.
+//   - The codes are read where they are: row-major int8 [n, k] of any k (no
+//     rewriting pass, no scratch), or the models' tiled format.
+//   - Optional prologue: the rows are the pre-normalisation rows of the
+//     LayerNorm before this linear (arctic.zig:716-746, 779-809), normalised
+//     on the way into LDS; the first column of blocks stores them.  A
+//     layer's LayerNorms then need no launch of their own.
+//   - Row scaling (SCALED: f32 rows of any magnitude): each row's largest
+//     magnitude in a chunk chooses the exponent e that puts it in [2^14,
+//     2^15), lowered (and the sums rescaled, exactly) by a later chunk that
+//     holds larger values, as gemm_pipe.hip does by stages.
+#include <type_traits>
+
+#include "pipe.h"
+
+namespace {
+
+enum { SE_BIAS = 0, SE_GELU = 1, SE_RES = 2 };  // SE_RES: + residual, stored f32 (a LayerNorm's input)
+
+struct SmallArgs {
+    const void *x;   // [m, k]
+    const void *w;   // codes: int8 [n, k] row-major, or W8T
+    const uint16_t *scale;
+    const float *bias;  // or null
+    void *c;            // [m, ldc]
+    const void *res;    // SE_RES: [m, n]
+    const float *gamma, *beta;  // LayerNorm prologue (k == 384)
+    float *xout;                // its rows [m, 384]
+    float eps;
+    int m, k, n, ldc;
+};
+
+#ifdef TZH_EMULATION
+inline int frexp_exp(float x) {
+    int e = 0;
+    if (std::isfinite(x)) std::frexp(x, &e);
+    return e;
+}
+inline float ldexp_f(float x, int e) { return std::ldexp(x, e); }
+#else
+__device__ __forceinline__ int frexp_exp(float x) { return __builtin_amdgcn_frexp_expf(x); }
+__device__ __forceinline__ float ldexp_f(float x, int e) { return __builtin_amdgcn_ldexpf(x, e); }
+#endif
+
+// Eight consecutive values of a row from column j; columns >= k are 0.
+template <typename TX>
+__device__ __forceinline__ void load_row8(const TX *row, int j, int k, TX (&v)[8]) {
+    if (j + 8 <= k) {
+        __builtin_memcpy(v, row + j, 8 * sizeof(TX));  // (16-byte loads; element alignment is enough)
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = j + i < k ? row[j + i] : (TX)0;
+    }
+}
+
+constexpr int kEUnset = 200;  // row exponent before any value: above every 15 - frexp_exp
+
+// BM rows by 16 NF WN outputs per block (NF fragments of 16 a wave), 4 / WN
+// waves over each chunk's k.
+template <typename TX, typename TC, typename TR, int EPI, bool WT, bool SCALED, bool LNP, int BM, int WN, int NF>
+__global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
+    constexpr bool SPLIT = sizeof(TX) == 4;
+    constexpr int WK = 4 / WN, KC = BM == 32 ? 512 : 1024, P = KC + 8, MF = BM / 16;
+    constexpr int TPR = 256 / BM;             // threads per row
+    constexpr int NP = KC / (8 * TPR);        // 8-value pieces per thread per chunk
+    constexpr int CS = KC / 64 / WK;          // 64-code groups of a wave per chunk
+    static_assert(WK == 1 || (MF == 1 && NF == 1), "shared k: one fragment to add up");
+    __shared__ __attribute__((aligned(16))) _Float16 xs[(SPLIT ? 2 : 1) * BM * P];
+    __shared__ int erow[SCALED ? BM : 1];
+    __shared__ __attribute__((aligned(16))) f32x4_t part[WK > 1 ? 256 : 1];
+    _Float16 *const xhi = xs, *const xlo = xs + (SPLIT ? BM * P : 0);
+
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int wn = WK == 1 ? w : 0, wk = WK == 1 ? 0 : w;
+    const int t0 = (int)blockIdx.y * BM, n0 = (int)blockIdx.x * (16 * NF * WN);
+    const int r16 = lane & 15, g = lane >> 4;
+    // this thread's row of X (clamped: rows past m repeat the last) and
+    // this lane's weight rows (past n: the last)
+    const int xr = tid / TPR, sub = tid % TPR;
+    const int trow = t0 + xr < a.m ? t0 + xr : a.m - 1;
+    const TX *const xrow = (const TX *)a.x + (size_t)trow * a.k;
+    int nrow[NF];
+#pragma unroll
+    for (int h = 0; h < NF; h++) {
+        const int nr = n0 + 16 * (NF * wn + h) + r16;
+        nrow[h] = nr < a.n ? nr : a.n - 1;
+    }
+
+    // codes k .. k + 15 of the lane's weight row, biased (u = q + 128).
+    // Codes at or past k multiply zeros; the loads stay inside the matrix.
+    auto load_codes = [&](int nrow, int k) __attribute__((always_inline)) {
+        typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+        if constexpr (WT) {
+            const size_t o = (((size_t)(nrow / 384) * (a.k / 64) + k / 64) * 384 + nrow % 384) * 64 + k % 64;
+            return *(const u32x4_t *)((const uint8_t *)a.w + o);
+        } else {
+            const uint8_t *const src = (const uint8_t *)a.w + (size_t)nrow * a.k + k;
+            u32x4_t v = {};
+            if ((size_t)nrow * a.k + k + 16 <= (size_t)a.n * a.k) {
+                __builtin_memcpy(&v, src, 16);
+            } else {
+                uint8_t b[16];
+#pragma unroll
+                for (int i = 0; i < 16; i++) b[i] = k + i < a.k ? src[i] : (uint8_t)0;
+                __builtin_memcpy(&v, b, 16);
+            }
+            return v ^ u32x4_t{0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};
+        }
+    };
+
+    f32x4_t acc[MF][NF];
+#pragma unroll
+    for (int f = 0; f < MF; f++)
+#pragma unroll
+        for (int h = 0; h < NF; h++) acc[f][h] = f32x4_t{};
+    int ecur = kEUnset;  // the thread's row's exponent
+    int eacc[MF];        // the exponent of acc[f]'s sums
+#pragma unroll
+    for (int f = 0; f < MF; f++) eacc[f] = kEUnset;
+
+    // 64-code groups of the chunk at c0, and this wave's: g0 .. g0 + gn - 1
+    auto groups_of = [&](int c0) __attribute__((always_inline)) {
+        return ((a.k - c0 < KC ? a.k - c0 : KC) + 63) / 64;
+    };
+    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+    struct Codes {
+        u32x4_t v[CS][NF];
+    } wc, wnext;
+    TX xv[NP][8];
+    auto load_chunk = [&](int c0, Codes &wd) __attribute__((always_inline)) {
+        const int groups = groups_of(c0), per = (groups + WK - 1) / WK, g0 = wk * per;
+        const int gn = groups - g0 < per ? groups - g0 : per;
+#pragma unroll
+        for (int s = 0; s < CS; s++)
+            if (s < gn)
+#pragma unroll
+                for (int h = 0; h < NF; h++) wd.v[s][h] = load_codes(nrow[h], c0 + 64 * (g0 + s) + 16 * g);
+#pragma unroll
+        for (int i = 0; i < NP; i++)
+            if (8 * TPR * i < 64 * groups) load_row8<TX>(xrow, c0 + 8 * (sub + TPR * i), a.k, xv[i]);
+    };
+    if constexpr (SPLIT) load_chunk(0, wc);
+    for (int c0 = 0; c0 < a.k; c0 += KC) {
+        if constexpr (!SPLIT) load_chunk(c0, wc);
+        const int groups = groups_of(c0), per = (groups + WK - 1) / WK, g0 = wk * per;
+        const int gn = groups - g0 < per ? groups - g0 : per;
+        if constexpr (LNP) {  // one chunk of 384 columns
+            float sum = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 384 / (8 * TPR); i++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) sum += (float)xv[i][e];
+#pragma unroll
+            for (int o = TPR / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+            const float mean = sum / 384.0f;
+            float sq = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 384 / (8 * TPR); i++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const float d = (float)xv[i][e] - mean;
+                    sq += d * d;
+                }
+#pragma unroll
+            for (int o = TPR / 2; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);
+            const float inv_std = 1.0f / sqrtf(sq / 384.0f + a.eps);
+#pragma unroll
+            for (int i = 0; i < 384 / (8 * TPR); i++) {
+                const int j = 8 * (sub + TPR * i);
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const f32x4_t gg = *(const f32x4_t *)(a.gamma + j + 4 * h), bb = *(const f32x4_t *)(a.beta + j + 4 * h);
+                    f32x4_t y;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        y[e] = (((float)xv[i][4 * h + e] - mean) * inv_std) * gg[e] + bb[e];
+                        xv[i][4 * h + e] = (TX)y[e];
+                    }
+                    if (blockIdx.x == 0 && t0 + xr < a.m) *(f32x4_t *)(a.xout + (size_t)trow * 384 + j + 4 * h) = y;
+                }
+            }
+        }
+        if constexpr (SCALED) {
+            float mx = 0.0f;
+#pragma unroll
+            for (int i = 0; i < NP; i++)
+                if (8 * TPR * i < 64 * groups)
+#pragma unroll
+                    for (int e = 0; e < 8; e++) mx = fmaxf(mx, fabsf((float)xv[i][e]));
+#pragma unroll
+            for (int o = TPR / 2; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+            if (mx > 0.0f) {
+                const int want = 15 - frexp_exp(mx);  // mx 2^want in [2^14, 2^15)
+                ecur = want < ecur ? want : ecur;
+            }
+        }
+        if (c0 > 0) __syncthreads();  // the last chunk's reads are done
+#pragma unroll
+        for (int i = 0; i < NP; i++)
+            if (8 * TPR * i < 64 * groups) {
+                const int o = xr * P + 8 * (sub + TPR * i);
+                if constexpr (SPLIT) {
+                    f32x4_t lo4, hi4;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        lo4[e] = SCALED ? ldexp_f((float)xv[i][e], ecur) : (float)xv[i][e];
+                        hi4[e] = SCALED ? ldexp_f((float)xv[i][4 + e], ecur) : (float)xv[i][4 + e];
+                    }
+                    half8_t h, l;
+                    split_f32x8(lo4, hi4, h, l);
+                    *(half8_t *)(xhi + o) = h;
+                    *(half8_t *)(xlo + o) = l;
+                } else {
+                    half8_t h;
+                    __builtin_memcpy(&h, xv[i], 16);
+                    *(half8_t *)(xhi + o) = h;
+                }
+            }
+        if constexpr (SCALED)
+            if (sub == 0) erow[xr] = ecur;
+        __syncthreads();
+        // f32: the next chunk's loads fly during this one's products (5 % at
+        // k = 1536; with f16 rows, at four blocks a CU, 5 % slower)
+        if constexpr (SPLIT)
+            if (c0 + KC < a.k) load_chunk(c0 + KC, wnext);
+        if constexpr (SCALED)
+#pragma unroll
+            for (int f = 0; f < MF; f++) {
+                const int e = erow[16 * f + r16];
+                if (e != eacc[f])
+#pragma unroll
+                    for (int h = 0; h < NF; h++)
+#pragma unroll
+                        for (int q = 0; q < 4; q++) acc[f][h][q] = ldexp_f(acc[f][h][q], e - eacc[f]);
+                eacc[f] = e;
+            }
+#pragma unroll
+        for (int s = 0; s < CS; s++)
+            if (s < gn) {
+                const int kk = 64 * (g0 + s) + 16 * g;
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    half8_t wf[NF];
+#pragma unroll
+                    for (int h = 0; h < NF; h++) wf[h] = codes_to_f16(wc.v[s][h][2 * j], wc.v[s][h][2 * j + 1]);
+#pragma unroll
+                    for (int f = 0; f < MF; f++) {
+                        const int o = (16 * f + r16) * P + kk + 8 * j;
+                        const half8_t xh = *(const half8_t *)(xhi + o);
+#pragma unroll
+                        for (int h = 0; h < NF; h++)
+                            acc[f][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[h], xh, acc[f][h], 0, 0, 0);
+                        if constexpr (SPLIT) {
+                            const half8_t xl = *(const half8_t *)(xlo + o);
+#pragma unroll
+                            for (int h = 0; h < NF; h++)
+                                acc[f][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[h], xl, acc[f][h], 0, 0, 0);
+                        }
+                    }
+                }
+            }
+        if constexpr (SPLIT) wc = wnext;
+    }
+
+    // lane (token r16, g) of fragments (f, h): outputs 4 g + e of 16
+    if constexpr (WK > 1) {
+        part[tid] = acc[0][0];
+        __syncthreads();
+        if (w > 0) return;
+#pragma unroll
+        for (int k = 1; k < WK; k++) acc[0][0] += part[64 * k + lane];
+    }
+#pragma unroll
+    for (int h = 0; h < NF; h++) {
+        const int n = n0 + 16 * (NF * wn + h) + 4 * g;
+        if (n >= a.n) continue;
+        float s[4], b[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int ne = n + e < a.n ? n + e : a.n - 1;
+            s[e] = f16_bits_to_f32(a.scale[ne]);
+            b[e] = a.bias ? a.bias[ne] : 0.0f;
+        }
+#pragma unroll
+        for (int f = 0; f < MF; f++) {
+            const int t = t0 + 16 * f + r16;
+            if (t >= a.m) continue;
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                v[e] = (SCALED ? ldexp_f(acc[f][h][e], -eacc[f]) : acc[f][h][e]) * s[e] + b[e];
+                if constexpr (EPI == SE_GELU) v[e] = gelu_fast(v[e]);
+            }
+            TC *const dst = (TC *)a.c + (size_t)t * a.ldc + n;
+            if (n + 4 <= a.n) {
+                if constexpr (EPI == SE_RES) {
+                    TR r[4];
+                    __builtin_memcpy(r, (const TR *)a.res + (size_t)t * a.n + n, 4 * sizeof(TR));
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[e] = (float)r[e] + v[e];
+                }
+                TC o[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) o[e] = (TC)v[e];
+                __builtin_memcpy(dst, o, 4 * sizeof(TC));
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (n + e < a.n)
+                        dst[e] = (TC)(EPI == SE_RES ? (float)((const TR *)a.res)[(size_t)t * a.n + n + e] + v[e] : v[e]);
+            }
+        }
+    }
+}
+
+template <typename TX, typename TC, typename TR, int EPI, bool WT, bool SCALED, bool LNP>
+int launch_small(hipStream_t st, int num_cus, const SmallArgs &a) {
+    // The largest tile that fills the chip: more outputs or rows a block
+    // share its rows' staging, its LDS reads and its code reads; 16 x 16
+    // tiles with shared k where even 16 x 64 would leave half the CUs idle
+    const int bn = (a.n + 63) / 64;
+    const int64_t rows16 = (a.m + 15) / 16, rows32 = (a.m + 31) / 32;
+    if (rows16 > 65535) return tzh_fail(TZH_ERR_TOO_LARGE, "internal: %d rows in the small linear", a.m);
+    if (rows32 * ((a.n + 127) / 128) >= num_cus) {
+        hipLaunchKernelGGL((linear_small_kernel<TX, TC, TR, EPI, WT, SCALED, LNP, 32, 4, 2>),
+                           dim3((unsigned)((a.n + 127) / 128), (unsigned)rows32), dim3(256), 0, st, a);
+    } else if (rows32 * bn >= num_cus) {
+        hipLaunchKernelGGL((linear_small_kernel<TX, TC, TR, EPI, WT, SCALED, LNP, 32, 4, 1>),
+                           dim3((unsigned)bn, (unsigned)rows32), dim3(256), 0, st, a);
+    } else if (rows16 * bn >= num_cus / 2) {
+        hipLaunchKernelGGL((linear_small_kernel<TX, TC, TR, EPI, WT, SCALED, LNP, 16, 4, 1>),
+                           dim3((unsigned)bn, (unsigned)rows16), dim3(256), 0, st, a);
+    } else {
+        hipLaunchKernelGGL((linear_small_kernel<TX, TC, TR, EPI, WT, SCALED, LNP, 16, 1, 1>),
+                           dim3((unsigned)((a.n + 15) / 16), (unsigned)rows16), dim3(256), 0, st, a);
+    }
+    TZH_LAUNCHED("linear_small_kernel");
+    return TZH_OK;
+}
+
+}  // namespace
+
+// Whether linear_small_kernel is the faster one for m rows: both times in us
+// as measured.  This kernel pays by the product (m n k in billions); the
+// pipelined one walks ceil(k / 64) serial stages once per 1536 columns
+// whatever m is, up to one round of tiles (beyond it this one has long
+// lost).  Measured, small / pipelined: f32 128 x 384 x 1152 5.2 / 27, 2048 x
+// 384 x 1536 GELU 20.8 / 30.4, 4096 x 384 x 1536 35 / 33, LayerNorm k = 1536
+// with 1024 rows 25 / 74, 8192 rows 73 / 76, 197 x 1000 x 1537 10 / 119;
+// f16 128 x 384 x 1152 4.0 / 14.9, 2048 x 384 x 1536 11.7 / 18.5, 4096 rows
+// 22 / 19.6, LayerNorm k = 1536 with 1024 rows 17 / 21, 2048 rows 27 / 22.
+bool tzh_linear_small_wins(int64_t m, int64_t k, int64_t n, bool f32, bool ln) {
+    if (m > 16384) return false;
+    const double work = (double)m * (double)k * (double)n * 1e-9, stages = (double)((k + 63) / 64);
+    const double launches = (double)((n + 1535) / 1536);
+    if (f32) return (ln ? 8.0 : 4.0) + 14.0 * work < launches * (6.0 + 3.0 * stages);
+    if (!ln) return 3.0 + 7.5 * work < launches * (8.0 + 1.3 * stages);
+    return 8.0 + 16.0 * work < (k > 384 ? 20.0 : 8.0 + 1.3 * stages);
+}
+
+// C = epi(X q^T s + b) for caller-owned codes q [n, k] (row-major int8, any
+// k >= 1), f32 (row-scaled) or f16 activations and output of the same type.
+// TZH_EPI_BIAS_RES_LN: pre_ln (f32 [m, n]) receives the rows before the
+// LayerNorm, residual added, and c is not written.
+int tzh_linear_small_launch(hipStream_t st, int num_cus, const void *x, int32_t x_dtype, const int8_t *q,
+                            const uint16_t *scale, const float *bias, void *c, int32_t c_dtype, int64_t m, int64_t k,
+                            int64_t n, int32_t epilogue, const void *res, float *pre_ln) {
+    SmallArgs a{};
+    a.x = x, a.w = q, a.scale = scale, a.bias = bias, a.res = res;
+    a.m = (int)m, a.k = (int)k, a.n = (int)n, a.ldc = (int)n;
+    a.c = epilogue == TZH_EPI_BIAS_RES_LN ? (void *)pre_ln : c;
+    const bool x32 = x_dtype == TZH_F32, c32 = c_dtype == TZH_F32;
+    auto typed = [&](auto tx, auto tc) -> int {
+        using TX = decltype(tx);
+        using TC = decltype(tc);
+        constexpr bool S = sizeof(TX) == 4;
+        switch (epilogue) {
+        case TZH_EPI_BIAS: return launch_small<TX, TC, TC, SE_BIAS, false, S, false>(st, num_cus, a);
+        case TZH_EPI_BIAS_GELU: return launch_small<TX, TC, TC, SE_GELU, false, S, false>(st, num_cus, a);
+        default: return launch_small<TX, float, TC, SE_RES, false, S, false>(st, num_cus, a);
+        }
+    };
+    if (x32) return c32 ? typed(0.0f, 0.0f) : typed(0.0f, (_Float16)0);
+    return c32 ? typed((_Float16)0, 0.0f) : typed((_Float16)0, (_Float16)0);
+}

@@ -1,7 +1,7 @@
 // Pipeline primitives shared by the kernels that stream operand tiles into
 // LDS with the gfx950 direct-to-LDS loads (gemm_pipe.hip, mlp.hip): the load
-// itself, the LDS-only workgroup barrier, explicit vmcnt waits, and the
-// tanh-form GELU of the bias epilogues.  The CPU emulation
+// itself, the LDS-only workgroup barrier, explicit vmcnt waits, the
+// tanh-form GELU of the bias epilogues and the widening of int8 codes.  The CPU emulation
 // (tests/cpu_emu/hip/hip_runtime.h) supplies its own dma16,
 // lds_barrier_only, vmem_*_issued and wave_lds_order.
 #pragma once
@@ -80,4 +80,25 @@ __device__ __forceinline__ float gelu_fast(float x) {
     constexpr float c1 = c0 * 0.044715f;
     const float e = __builtin_amdgcn_exp2f(x * __builtin_fmaf(x * x, c1, c0));
     return x * __builtin_amdgcn_rcpf(e + 1.0f);
+}
+
+// Eight biased int8 weight codes (u = q + 128, little-endian in d0, d1) ->
+// f16 q, exactly: v_perm_b32 makes each code the low mantissa byte of an f16
+// with exponent 10 (bits 0x64uu = 1024 + u), and a packed f16 subtraction of
+// 1152 = 1024 + 128 leaves q; every value is an integer below 2048, so
+// nothing rounds.
+__device__ __forceinline__ half8_t codes_to_f16(uint32_t d0, uint32_t d1) {
+    const half2_t off = {(_Float16)1152.0f, (_Float16)1152.0f};
+    half8_t r;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const uint32_t d = i ? d1 : d0;
+        const half2_t lo = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, d, 0x04010400u)) - off;
+        const half2_t hi = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, d, 0x04030402u)) - off;
+        r[4 * i + 0] = lo[0];
+        r[4 * i + 1] = lo[1];
+        r[4 * i + 2] = hi[0];
+        r[4 * i + 3] = hi[1];
+    }
+    return r;
 }

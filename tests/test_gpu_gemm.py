@@ -362,3 +362,46 @@ def test_layernorm_entry_vs_oracle(ctx):
     check(lib().tzh_layernorm_last_dim(ctx.handle, X.data_ptr(), G.data_ptr(), B.data_ptr(), X.data_ptr(), 300, 384,
                                        1e-12))  # in place (layernorm.zig:26-35 allows input == output)
     np.testing.assert_allclose(X.cpu().numpy(), ref, rtol=1e-5, atol=2e-5)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("m,k,n,epi", [
+    (1, 1, 384, _abi.EPI_BIAS), (15, 63, 384, _abi.EPI_BIAS), (17, 65, 768, _abi.EPI_BIAS_GELU),   # 16 x 16 tiles, shared k
+    (16, 1024, 384, _abi.EPI_BIAS_RES_LN), (5, 1025, 384, _abi.EPI_BIAS_RES_LN), (3, 2049, 384, _abi.EPI_BIAS),
+    (300, 511, 384, _abi.EPI_BIAS), (129, 513, 1536, _abi.EPI_BIAS_GELU), (500, 1600, 384, _abi.EPI_BIAS_RES_LN),
+    (1501, 385, 768, _abi.EPI_BIAS), (1030, 512, 1152, _abi.EPI_BIAS)])  # 32-row tiles, one and two fragments a wave
+def test_few_row_linear(ctx, m, k, n, epi, dtype):
+    """The few-row kernel at the edges of its tiles and k chunks, every
+    epilogue, f32 and f16, against float64 (f16: the products are exact, the
+    output rounds once; GELU and LayerNorm as their own tests bound them)."""
+    a, q, s, bias = make_problem(m * 7 + k + n, m, k, n)
+    q[:, k // 2] = 0
+    a[m // 2] = 0.0  # a row without a largest magnitude
+    a = a.astype(dtype)
+    rng = np.random.default_rng(m)
+    res = rng.standard_normal((m, n)).astype(dtype)
+    g, b = (1 + 0.1 * rng.standard_normal(n)).astype(np.float32), (0.1 * rng.standard_normal(n)).astype(np.float32)
+    A, Q, S, B, R, G, Bt = dev(a), dev(q), dev(s.view(np.int16)), dev(bias), dev(res), dev(g), dev(b)
+    code = _abi.F32 if dtype == np.float32 else _abi.F16
+    out = torch.empty((m, n), dtype=torch.float32 if dtype == np.float32 else torch.float16, device="cuda")
+    check(lib().tzh_linear_w8(ctx.handle, A.data_ptr(), code, Q.data_ptr(), S.data_ptr(), B.data_ptr(), out.data_ptr(),
+                              code, m, k, n, epi, R.data_ptr(), code, G.data_ptr(), Bt.data_ptr(), 1e-12))
+    got = out.cpu().numpy().astype(np.float64)
+    sf = s.view(np.float16).astype(np.float64)
+    lin = (a.astype(np.float64) @ q.astype(np.float64).T) * sf + bias
+    half = 0.0 if dtype == np.float32 else 2.0 ** -11
+    tol = bound(a.astype(np.float32), q, s, lin, k)
+    if epi == _abi.EPI_BIAS:
+        assert (np.abs(got - lin) <= tol + half * np.abs(lin) + 2.0 ** -24).all()
+        return
+    if epi == _abi.EPI_BIAS_GELU:
+        ref = 0.5 * lin * (1 + np.tanh(0.7978845608 * (lin + 0.044715 * lin ** 3)))
+        assert (np.abs(got - ref) <= 1.2 * tol + (half + 2.0 ** -20) * np.abs(ref) + 2e-6).all()
+        return
+    v = res.astype(np.float64) + lin
+    mean, std = v.mean(1, keepdims=True), v.std(1, keepdims=True)
+    ref = (v - mean) / std * g + b
+    # an error d of the pre-norm values moves the normalised ones by at most
+    # about 2 d / std (their mean and deviation move with them), times gamma
+    bar = 1.5 * (2 * tol.max(1, keepdims=True) / std + 2.0 ** -20 * (1 + np.abs(ref))) + half * np.abs(ref) + 2.0 ** -24
+    assert (np.abs(got - ref) <= bar).all()
