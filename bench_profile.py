@@ -65,7 +65,7 @@ def stage_of(kernel: str, prev: str | None) -> str | None:
     """Forward stage of a dispatch of `kernel`, given the previous stage."""
     if "pack_ids_kernel" in kernel:
         return "pack_ids"
-    if "embed_ln_kernel" in kernel:
+    if "embed_ln_kernel" in kernel or "embed_ids_ln_kernel" in kernel:
         return "embed_ln"
     if "attn_varlen_kernel" in kernel or "attn_varlen_f32_kernel" in kernel:
         return "attention"
@@ -106,8 +106,8 @@ def _rows(directory: str, suffix: str) -> list[dict]:
 def _instances(seq):
     """Groups (kernel name, value) dispatches in launch order into stage
     instances per forward precision: {"fp32" | "fp16": {stage: [summed
-    value of each instance]}}.  A forward runs from one pack_ids dispatch to
-    the next; its precision is that of its attention kernel.  A dispatch that
+    value of each instance]}}.  A forward runs from one pack_ids or
+    embed_ids_ln_kernel dispatch (up to 256 sequences) to the next; its precision is that of its attention kernel.  A dispatch that
     continues the previous stage (the pieces of a split LayerNorm round, the
     fused kernel's split-round rows) adds to that stage's current instance.  Forwards that launch a stage
     twice in a row (bench.py's per-launch timing forwards repeat each stage)
@@ -126,7 +126,7 @@ def _instances(seq):
         st = stage_of(name, prev)
         if st is None:
             continue
-        if st == "pack_ids":
+        if st == "pack_ids" or "embed_ids_ln_kernel" in name:
             flush()
             fwd, prec, repeated = {}, None, False
         if st == "attention":
@@ -194,8 +194,8 @@ def kernel_stats_table(directory: str, top: int = 10) -> list[str]:
 
 def forward_sum_us(stages: dict) -> float | None:
     """Kernel time of one forward: every stage's average times its launches
-    per forward (pack_ids runs once per forward)."""
-    n_fwd = (stages.get("pack_ids") or {}).get("instances") or 0
+    per forward (embed_ln runs once per forward)."""
+    n_fwd = (stages.get("embed_ln") or {}).get("instances") or 0
     if not n_fwd:
         return None
     return sum(v["avg_us"] * v["instances"] / n_fwd for v in stages.values() if v["instances"] and v["avg_us"])

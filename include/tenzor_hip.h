@@ -443,7 +443,8 @@ int tzh_arctic_precision(tzh_model *model, int32_t *dtype);
  * 1536-wide intermediate kept on chip (its last, partial round of 64-token
  * panels split by chunks over the idle CUs and finished by a second, small
  * kernel), unless the model's weights call for row scaling; other layers
- * run the GEMM pair. */
+ * run the GEMM pair.  A few hundred tokens run the two linears and the
+ * LayerNorm as three launches of many small blocks instead. */
 int tzh_arctic_feed_forward(tzh_model *model, int32_t layer, const float *input, float *output, int64_t seq_len);
 
 /* Fused feed-forward switch (no counterpart in the reference): enable = 0
@@ -457,7 +458,7 @@ int tzh_arctic_set_ffn_fusion(tzh_model *model, int32_t enable);
 /* Launch tracing (no counterpart in the reference, whose CPU path has no
  * kernels to time): with timing enabled (enable = n >= 1), every later
  * forward records a HIP event on the model's stream before its first and
- * after each of its stages, and issues each stage after pack_ids n times
+ * after each of its stages, and issues each stage after the first n times
  * back to back between its events (every such stage reads only buffers it
  * does not write, so the result is unchanged), which spreads the cost of
  * an event over n launches.  enable = 0 turns it off; n <= 1000. */
@@ -466,11 +467,14 @@ int tzh_arctic_set_timing(tzh_model *model, int32_t enable);
 /* Per-launch durations of the most recent timed forward, in launch order:
  * us[i] (microseconds between the events around stage i, divided by the
  * times it was issued) and names[i]
- * (static stage names: "pack_ids", "embed_ln", "qkv", "attention",
+ * (static stage names: "pack_ids" (batches of over 256 sequences),
+ * "embed_ln", "qkv", "attention",
  * "attn_out_ln" and "ffn" (the fused feed-forward kernel), or "attn_ffn"
  * (the O-projection, its LayerNorm and the feed-forward block as one
  * kernel; both fused stages include the kernel that finishes the rows of a
- * split last round), or "attn_out_ln", "ffn1_gelu" and "ffn2_ln" (the GEMM pair),
+ * split last round), or "attn_out_ln", "ffn1_gelu" and "ffn2_ln" (the GEMM
+ * pair; in forwards of a few hundred tokens each LayerNorm runs at the head
+ * of the stage after),
  * "cls_l2", "hidden_f32"), at most
  * `capacity` entries; *count = number of launches (0 if the last forward was
  * not timed).  Waits for that forward to finish.  Either array may be NULL. */

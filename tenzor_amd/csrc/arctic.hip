@@ -29,6 +29,11 @@
 #include "safetensors.h"
 #include "tenzor_file.h"
 
+int64_t tzh_small_layer_rows(int num_cus);
+int64_t tzh_small_ffn_rows(int num_cus);
+int tzh_linear_small_model_launch(hipStream_t st, int num_cus, const float *x, const float *gamma, const float *beta,
+                                  float eps, float *xout, const void *w, const uint16_t *scale, const float *bias,
+                                  float *c, int64_t m, int64_t k, int64_t n, int32_t epilogue, const float *res);
 int tzh_linear_codes_launch(hipStream_t st, int num_cus, const void *x, int32_t x_dtype, const void *wc,
                             int32_t w_format, const uint16_t *scale, const float *bias, void *c, int32_t c_dtype,
                             int64_t m, int64_t k, int64_t n, int64_t n_valid, int32_t epilogue, const void *res,
@@ -90,17 +95,10 @@ struct TableRef {
 // K2: x = (word[id] + pos[p]) + type[0], then LayerNorm (arctic.zig:543-585).
 // One wave per token, six columns per lane.
 template <typename TO>
-__global__ void __launch_bounds__(256) embed_ln_kernel(const uint32_t *__restrict__ tok_ids,
-                                                       const int32_t *__restrict__ tok_pos, int64_t T,
-                                                       TableRef word, TableRef pos, TableRef type,
-                                                       const float *__restrict__ gamma,
-                                                       const float *__restrict__ beta, float eps,
-                                                       TO *__restrict__ out) {
-    const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+__device__ __forceinline__ void embed_row(int64_t t, int64_t id, int64_t p, const TableRef &word, const TableRef &pos,
+                                          const TableRef &type, const float *gamma, const float *beta, float eps,
+                                          TO *out) {
     const int lane = threadIdx.x & 63;
-    if (t >= T) return;
-    const int64_t id = tok_ids[t];
-    const int64_t p = tok_pos[t];
     float x[6];
     float sum = 0.0f;
 #pragma unroll
@@ -127,6 +125,50 @@ __global__ void __launch_bounds__(256) embed_ln_kernel(const uint32_t *__restric
     }
 }
 
+template <typename TO>
+__global__ void __launch_bounds__(256) embed_ln_kernel(const uint32_t *__restrict__ tok_ids,
+                                                       const int32_t *__restrict__ tok_pos, int64_t T,
+                                                       TableRef word, TableRef pos, TableRef type,
+                                                       const float *__restrict__ gamma,
+                                                       const float *__restrict__ beta, float eps,
+                                                       TO *__restrict__ out) {
+    const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (t >= T) return;
+    embed_row<TO>(t, tok_ids[t], tok_pos[t], word, pos, type, gamma, beta, eps, out);
+}
+
+// The same from the caller's ids, with the batch's offsets and attention
+// order as kernel arguments (up to kMetaBatch sequences): block (x, b) takes
+// tokens 4 x .. 4 x + 3 of sequence b, and the first block stores the
+// offsets and the order for the kernels after it.  A small forward so
+// starts with one launch instead of a copy, the id packing and this
+// (about 8 of its first 10 us).
+constexpr int kMetaBatch = 256;
+struct BatchMeta {
+    int v[2 * kMetaBatch + 1];  // cu[batch + 1], order[batch]
+};
+template <typename TO>
+__global__ void __launch_bounds__(256) embed_ids_ln_kernel(const uint32_t *__restrict__ ids, int64_t stride, int batch,
+                                                           const BatchMeta meta, int *__restrict__ meta_out,
+                                                           uint32_t vocab, int *__restrict__ bad, TableRef word,
+                                                           TableRef pos, TableRef type,
+                                                           const float *__restrict__ gamma,
+                                                           const float *__restrict__ beta, float eps,
+                                                           TO *__restrict__ out) {
+    const int b = blockIdx.y;
+    if (blockIdx.x == 0 && b == 0)
+        for (int i = threadIdx.x; i < 2 * batch + 1; i += 256) meta_out[i] = meta.v[i];
+    const int start = meta.v[b], L = meta.v[b + 1] - start;
+    const int j = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (j >= L) return;
+    uint32_t id = (stride ? ids + (int64_t)b * stride : ids + start)[j];
+    if (id >= vocab) {  // counted, clamped to keep the gather in bounds
+        if ((threadIdx.x & 63) == 0) atomicAdd(bad, 1);
+        id = vocab - 1;
+    }
+    embed_row<TO>(start + j, id, j, word, pos, type, gamma, beta, eps, out);
+}
+
 // K5: CLS row of every sequence, L2-normalised (arctic.zig:893-897, 851-863).
 template <typename TI>
 __global__ void __launch_bounds__(256) cls_l2_kernel(const TI *__restrict__ hidden, const int *__restrict__ cu,
@@ -139,6 +181,38 @@ __global__ void __launch_bounds__(256) cls_l2_kernel(const TI *__restrict__ hidd
 #pragma unroll
     for (int q = 0; q < 6; q++) {
         v[q] = (float)row[lane + 64 * q];
+        ss += v[q] * v[q];
+    }
+    const float norm = sqrtf(wave_sum(ss));
+#pragma unroll
+    for (int q = 0; q < 6; q++) out[(int64_t)b * H + lane + 64 * q] = norm > 1e-12f ? v[q] / norm : v[q];
+}
+
+// The same from the rows before the encoder's last LayerNorm, normalised
+// first (the few-row forward).
+__global__ void __launch_bounds__(256) cls_ln_l2_kernel(const float *__restrict__ rows, const int *__restrict__ cu,
+                                                        int batch, const float *__restrict__ gamma,
+                                                        const float *__restrict__ beta, float eps,
+                                                        float *__restrict__ out) {
+    const int b = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (b >= batch) return;
+    const float *row = rows + (int64_t)cu[b] * H;
+    float v[6], s = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 6; q++) {
+        v[q] = row[lane + 64 * q];
+        s += v[q];
+    }
+    const float mean = wave_sum(s) / (float)H;
+    float vs = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 6; q++) vs += (v[q] - mean) * (v[q] - mean);
+    const float inv_std = 1.0f / sqrtf(wave_sum(vs) / (float)H + eps);
+    float ss = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 6; q++) {
+        v[q] = ((v[q] - mean) * inv_std) * gamma[lane + 64 * q] + beta[lane + 64 * q];
         ss += v[q] * v[q];
     }
     const float norm = sqrtf(wave_sum(ss));
@@ -499,6 +573,22 @@ int layernorm_rows(hipStream_t st, const float *x, const float *g, const float *
 // an f32 second linear writes its pre-norm rows to the workspace's attn).
 bool ffn_fused(const tzh_model *m, const DevLayer &d, int32_t act, bool rs) {
     return m->fuse_ffn && d.mlp && act == TZH_F32 && !rs;
+}
+
+// Whether layer d's linears of T rows run one by one on the few-row kernel
+// (all int8, f32 activations inside the split's range).
+bool small_layer(const tzh_model *m, const DevLayer &d, int32_t act, bool rs, int64_t T) {
+    return m->fuse_ffn && act == TZH_F32 && !rs && T <= tzh_small_layer_rows(m->ctx->num_cus) && d.qkv.fmt == TZH_WF_W8T &&
+           d.o.fmt == TZH_WF_W8T && d.ffn1.fmt == TZH_WF_W8T && d.ffn2.fmt == TZH_WF_W8T;
+}
+
+// One such linear: y = epi(x W^T s + b), x optionally normalised on the way
+// in (ln_g, ln_b) with the normalised rows stored to xout.
+int small_linear(const tzh_model *m, hipStream_t st, const DevLinear &l, const float *x, float *y, int64_t T, int64_t k,
+                 int64_t n, int32_t epilogue, const float *res, const float *ln_g = nullptr,
+                 const float *ln_b = nullptr, float *xout = nullptr) {
+    return tzh_linear_small_model_launch(st, m->ctx->num_cus, x, ln_g, ln_b, m->cfg.layer_norm_eps, xout, l.w, l.s, l.b,
+                                         y, T, k, n, epilogue, res);
 }
 
 int ffn_part(tzh_model *m, const DevLayer &d, hipStream_t st, int32_t act, bool rs, const void *x, void *y, int64_t T,
@@ -932,15 +1022,20 @@ int run_forward(tzh_model *m, float *outputs, float *hidden_out, const uint32_t 
     TZH_TRY(ensure_workspace(m, T, batch, es));
     hipStream_t st = m->ctx->stream;
 
-    // metadata: cu_seqlens and a longest-first order for attention
-    TZH_HIP(hipEventSynchronize(m->meta_done));  // previous copy out of the staging buffer finished
-    int *cu = m->host_meta, *order = m->host_meta + batch + 1;
+    // metadata: cu_seqlens and a longest-first order for attention; few
+    // sequences' travel as arguments of the first kernel
+    BatchMeta arg;
+    const bool by_arg = batch <= kMetaBatch;
+    if (!by_arg) TZH_HIP(hipEventSynchronize(m->meta_done));  // previous copy out of the staging buffer finished
+    int *cu = by_arg ? arg.v : m->host_meta, *order = cu + batch + 1;
     cu[0] = 0;
     for (int b = 0; b < batch; b++) cu[b + 1] = cu[b] + lengths[b];
     std::iota(order, order + batch, 0);
     std::stable_sort(order, order + batch, [&](int x, int y) { return lengths[x] > lengths[y]; });
-    TZH_HIP(hipMemcpyAsync(m->meta, m->host_meta, (size_t)(2 * batch + 1) * 4, hipMemcpyHostToDevice, st));
-    TZH_HIP(hipEventRecord(m->meta_done, st));
+    if (!by_arg) {
+        TZH_HIP(hipMemcpyAsync(m->meta, m->host_meta, (size_t)(2 * batch + 1) * 4, hipMemcpyHostToDevice, st));
+        TZH_HIP(hipEventRecord(m->meta_done, st));
+    }
     const int *d_cu = m->meta, *d_order = m->meta + batch + 1;
 
     int launches = 0;
@@ -973,10 +1068,25 @@ int run_forward(tzh_model *m, float *outputs, float *hidden_out, const uint32_t 
         }
         TZH_HIP(hipEventRecord(m->events[0], st));
     }
-    hipLaunchKernelGGL(pack_ids_kernel, dim3(batch), dim3(256), 0, st, ids, ids_stride, d_cu, m->tok_ids, m->tok_pos,
-                       (uint32_t)m->cfg.vocab_size, m->bad_ids);
-    TZH_LAUNCHED("pack_ids_kernel");
-    TZH_TRY(mark("pack_ids"));
+    if (by_arg) {
+        // (once, whatever the timing repetitions: it counts clamped ids)
+        const dim3 grid((unsigned)((lengths[order[0]] + 3) / 4), (unsigned)batch);
+        if (act == TZH_F32)
+            hipLaunchKernelGGL(embed_ids_ln_kernel<float>, grid, dim3(256), 0, st, ids, ids_stride, batch, arg, m->meta,
+                               (uint32_t)m->cfg.vocab_size, m->bad_ids, m->word.ref(), m->pos.ref(), m->type.ref(),
+                               m->emb_g, m->emb_b, m->cfg.layer_norm_eps, (float *)m->h);
+        else
+            hipLaunchKernelGGL(embed_ids_ln_kernel<_Float16>, grid, dim3(256), 0, st, ids, ids_stride, batch, arg,
+                               m->meta, (uint32_t)m->cfg.vocab_size, m->bad_ids, m->word.ref(), m->pos.ref(),
+                               m->type.ref(), m->emb_g, m->emb_b, m->cfg.layer_norm_eps, (_Float16 *)m->h);
+        TZH_LAUNCHED("embed_ids_ln_kernel");
+        TZH_TRY(mark("embed_ln"));
+    } else {
+        hipLaunchKernelGGL(pack_ids_kernel, dim3(batch), dim3(256), 0, st, ids, ids_stride, d_cu, m->tok_ids, m->tok_pos,
+                           (uint32_t)m->cfg.vocab_size, m->bad_ids);
+        TZH_LAUNCHED("pack_ids_kernel");
+        TZH_TRY(mark("pack_ids"));
+    }
     // Every later stage reads buffers that it does not write, so issuing it
     // again gives the same result: with timing on, each is issued
     // timing_reps times between its events (pack_ids, which counts
@@ -986,7 +1096,7 @@ int run_forward(tzh_model *m, float *outputs, float *hidden_out, const uint32_t 
         for (int r = 0; r < reps; r++) TZH_TRY(launch());
         return mark(name, reps);
     };
-    TZH_TRY(stage("embed_ln", [&]() -> int {
+    if (!by_arg) TZH_TRY(stage("embed_ln", [&]() -> int {
         if (act == TZH_F32)
             hipLaunchKernelGGL(embed_ln_kernel<float>, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, st, m->tok_ids,
                                m->tok_pos, T, m->word.ref(), m->pos.ref(), m->type.ref(), m->emb_g, m->emb_b,
@@ -999,6 +1109,9 @@ int run_forward(tzh_model *m, float *outputs, float *hidden_out, const uint32_t 
         return TZH_OK;
     }));
     const float eps = m->cfg.layer_norm_eps;
+    bool small = n_layers > 0;
+    for (int32_t li = 0; li < n_layers; li++)
+        small = small && small_layer(m, m->layers[(size_t)li], act, m->row_scaled, T);
     for (int32_t li = 0; li < n_layers; li++) {
         const DevLayer &d = m->layers[(size_t)li];
         const int cus = m->ctx->num_cus;
@@ -1013,6 +1126,33 @@ int run_forward(tzh_model *m, float *outputs, float *hidden_out, const uint32_t 
                 return tzh_fail(TZH_ERR_INVALID_ARGS, "layer %d: weight format %d cannot run with activation type %d", li,
                                 l->fmt, act);
         float *const hf = (float *)m->h, *const h1f = (float *)m->h1;
+        if (small) {
+            // five launches a layer: h1 holds the rows before each LayerNorm,
+            // which the linear reading them normalises (into h, the
+            // residual of the one after)
+            const DevLayer *const prev = li ? &m->layers[(size_t)li - 1] : nullptr;
+            float *const inter = (float *)m->inter;
+            TZH_TRY(stage("qkv", [&]() {
+                return prev ? small_linear(m, st, d.qkv, h1f, (float *)m->qkv, T, H, 3 * H, TZH_EPI_BIAS, nullptr,
+                                           prev->ln2_g, prev->ln2_b, hf)
+                            : small_linear(m, st, d.qkv, hf, (float *)m->qkv, T, H, 3 * H, TZH_EPI_BIAS, nullptr);
+            }));
+            TZH_TRY(stage("attention", [&]() {
+                return tzh_attention_launch(st, cus, m->ctx->work_queue, m->qkv, m->attn, act, d_cu, d_order, batch, 12,
+                                            H);
+            }));
+            TZH_TRY(stage("attn_out_ln", [&]() {
+                return small_linear(m, st, d.o, (const float *)m->attn, h1f, T, H, H, TZH_EPI_BIAS_RES_LN, hf);
+            }));
+            TZH_TRY(stage("ffn1_gelu", [&]() {
+                return small_linear(m, st, d.ffn1, h1f, inter, T, H, 1536, TZH_EPI_BIAS_GELU, nullptr, d.ln1_g, d.ln1_b,
+                                    hf);
+            }));
+            TZH_TRY(stage("ffn2_ln", [&]() {
+                return small_linear(m, st, d.ffn2, inter, h1f, T, 1536, H, TZH_EPI_BIAS_RES_LN, hf);
+            }));
+            continue;
+        }
         // row-scaled int8 GEMMs when the weights do not bound their inputs
         // inside the split's range (set_range)
         const bool rs = m->row_scaled && act == TZH_F32;
@@ -1059,9 +1199,14 @@ int run_forward(tzh_model *m, float *outputs, float *hidden_out, const uint32_t 
             TZH_TRY(stage("ffn2_ln", [&]() { return ffn_part(m, d, st, act, rs, m->h1, m->h, T, 2); }));
         }
     }
+    // the last LayerNorm of a few-row forward has no linear to do it
+    const DevLayer *const last = small ? &m->layers[(size_t)n_layers - 1] : nullptr;
     if (outputs) {
         TZH_TRY(stage("cls_l2", [&]() -> int {
-            if (act == TZH_F32)
+            if (last)
+                hipLaunchKernelGGL(cls_ln_l2_kernel, dim3((unsigned)((batch + 3) / 4)), dim3(256), 0, st,
+                                   (const float *)m->h1, d_cu, batch, last->ln2_g, last->ln2_b, eps, outputs);
+            else if (act == TZH_F32)
                 hipLaunchKernelGGL(cls_l2_kernel<float>, dim3((unsigned)((batch + 3) / 4)), dim3(256), 0, st,
                                    (const float *)m->h, d_cu, batch, outputs);
             else
@@ -1073,7 +1218,9 @@ int run_forward(tzh_model *m, float *outputs, float *hidden_out, const uint32_t 
     }
     if (hidden_out) {
         const int64_t n = T * H;
-        if (act == TZH_F32) {
+        if (last) {
+            TZH_TRY(layernorm_rows(st, (const float *)m->h1, last->ln2_g, last->ln2_b, hidden_out, T, H, eps));
+        } else if (act == TZH_F32) {
             TZH_HIP(hipMemcpyAsync(hidden_out, m->h, (size_t)n * 4, hipMemcpyDeviceToDevice, st));
         } else {
             hipLaunchKernelGGL(f16_to_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
@@ -1215,6 +1362,16 @@ extern "C" int tzh_arctic_feed_forward(tzh_model *m, int32_t layer, const float 
     const DevLayer &d = m->layers[(size_t)layer];
     const bool rs = m->row_scaled;
     hipStream_t st = m->ctx->stream;
+    // few rows: the two linears on the few-row kernel (the intermediate and
+    // the rows before the LayerNorm in the fused kernel's scratch)
+    const size_t need = (size_t)seq_len * (1536 + H) * 4;
+    if (seq_len <= tzh_small_ffn_rows(m->ctx->num_cus) && small_layer(m, d, TZH_F32, rs, seq_len) &&
+        need <= m->mlp_tail_bytes) {
+        float *const inter = (float *)m->mlp_tail, *const rows = inter + (size_t)seq_len * 1536;
+        TZH_TRY(small_linear(m, st, d.ffn1, input, inter, seq_len, H, 1536, TZH_EPI_BIAS_GELU, nullptr));
+        TZH_TRY(small_linear(m, st, d.ffn2, inter, rows, seq_len, 1536, H, TZH_EPI_BIAS_RES_LN, input));
+        return layernorm_rows(st, rows, d.ln2_g, d.ln2_b, output, seq_len, H, m->cfg.layer_norm_eps);
+    }
     if (ffn_fused(m, d, TZH_F32, rs)) return ffn_part(m, d, st, TZH_F32, rs, input, output, seq_len, 0);
     TZH_TRY(ensure_workspace(m, seq_len, 1, 4));
     TZH_TRY(ffn_part(m, d, st, TZH_F32, rs, input, output, seq_len, 1));

@@ -233,7 +233,9 @@ __global__ void __launch_bounds__(NW * 64) attn_varlen_kernel(const _Float16 *__
 // That removes about 12 of 78 VALU ops per block (1 % faster).
 constexpr int kWavesF32 = 16;
 
-template <int NW>
+// PARTS > 1: the query tiles of an item are dealt to PARTS blocks, each of
+// which stages all its keys: for batches whose items leave most CUs idle.
+template <int NW, int PARTS>
 __global__ void __launch_bounds__(NW * 64) attn_varlen_f32_kernel(const float *__restrict__ qkv, int ld,
                                                               float *__restrict__ out, int ld_out,
                                                               const int *__restrict__ cu_seqlens,
@@ -254,7 +256,7 @@ __global__ void __launch_bounds__(NW * 64) attn_varlen_f32_kernel(const float *_
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int g = lane >> 4, ql = lane & 15;
     const int gq = lane & 3, dp = lane >> 2;  // V staging: slot group, dim pair
-    const int n_items = batch * n_heads;
+    const int n_items = batch * n_heads * PARTS;
 
     // Persistent blocks over items (item j: the j / n_heads-th sequence of
     // `order`, longest first, head j % n_heads).  Block b starts with item b
@@ -264,14 +266,15 @@ __global__ void __launch_bounds__(NW * 64) attn_varlen_f32_kernel(const float *_
     // queries run, so a block's loads overlap its MFMA work: with one 145 KiB
     // workgroup per CU nothing else would hide them.
     struct Item {
-        int start, L, h;
+        int start, L, h, part;
     };
-    auto item_of = [&](int j) {
+    auto item_of = [&](int jp) {
+        const int j = jp / PARTS, part = jp % PARTS;
         const int s = j / n_heads;
         const int b = order ? order[s] : s;
         const int start = cu_seqlens[b];
         // the host validates lengths; the clamp keeps every LDS index in bounds regardless
-        return Item{start, min(max(cu_seqlens[b + 1] - start, 0), kMaxKeys), j % n_heads};
+        return Item{start, min(max(cu_seqlens[b + 1] - start, 0), kMaxKeys), j % n_heads, part};
     };
     // prefetch registers: K units u = tid + 1024 i (key u / 4, dims 8 (u % 4)
     // + [0, 8)) and V keys 32 w + 4 gq + (r % 4) + 16 (r / 4), dims 2 dp and
@@ -367,7 +370,7 @@ __global__ void __launch_bounds__(NW * 64) attn_varlen_f32_kernel(const float *_
             }
         };
         f32x4_t qa = {0, 0, 0, 0}, qb = {0, 0, 0, 0};
-        load_q(16 * w, qa, qb);
+        load_q(16 * (w * PARTS + cur.part), qa, qb);
         stage(cur);
         __syncthreads();
         // Q is split before the next item's loads are issued, so that its
@@ -376,11 +379,11 @@ __global__ void __launch_bounds__(NW * 64) attn_varlen_f32_kernel(const float *_
         half8_t qh, qlo;
         split_f32x8(qa * scale4, qb * scale4, qh, qlo);
         const int jn = next_item;  // written before the barrier above, rewritten after the one below
-        const Item nxt = jn < n_items ? item_of(jn) : Item{0, 0, 0};
+        const Item nxt = jn < n_items ? item_of(jn) : Item{0, 0, 0, 0};
         prefetch(nxt);
 
         for (int t2 = 0; t2 < 2; t2++) {
-            const int q0 = 16 * (w + NW * t2);
+            const int q0 = 16 * ((w + NW * t2) * PARTS + cur.part);
             if (q0 >= L) break;
             const int qrow = q0 + ql;
             if (t2) {
@@ -535,10 +538,24 @@ int tzh_attention_launch(hipStream_t st, int num_cus, unsigned *queue, const voi
     if (dtype == TZH_F32) {
         if (!queue) return tzh_fail(TZH_ERR_INVALID_ARGS, "internal: attention without its work queue");
         if ((int64_t)batch * n_heads > INT32_MAX) return tzh_fail(TZH_ERR_TOO_LARGE, "attention: too many (sequence, head) items");
-        const int64_t blocks = std::min<int64_t>((int64_t)batch * n_heads, std::max(num_cus, 1));
-        hipLaunchKernelGGL((attn_varlen_f32_kernel<kWavesF32>), dim3((unsigned)blocks), dim3(kWavesF32 * 64), 0, st,
-                           (const float *)qkv, 3 * hidden, (float *)out, hidden, cu_seqlens, order, batch, n_heads,
-                           hidden, scale_log2, queue);
+        // Few items: their query tiles over up to 8 blocks each while every
+        // block has a CU of its own.  Measured (12 heads, us a call, of which
+        // 17 are the entry point's check of the lengths): one sequence of 512
+        // 47 -> 31 and two 48 -> 33 (8 parts), ten of 16 to 512 49 -> 40 (2);
+        // of 128 tokens no change.
+        const int64_t items = (int64_t)batch * n_heads, cus = std::max(num_cus, 1);
+        const dim3 block(kWavesF32 * 64);
+        const float *const q = (const float *)qkv;
+        float *const o = (float *)out;
+        if (items * 8 <= cus)
+            hipLaunchKernelGGL((attn_varlen_f32_kernel<kWavesF32, 8>), dim3((unsigned)(items * 8)), block, 0, st, q,
+                               3 * hidden, o, hidden, cu_seqlens, order, batch, n_heads, hidden, scale_log2, queue);
+        else if (items * 2 <= cus)
+            hipLaunchKernelGGL((attn_varlen_f32_kernel<kWavesF32, 2>), dim3((unsigned)(items * 2)), block, 0, st, q,
+                               3 * hidden, o, hidden, cu_seqlens, order, batch, n_heads, hidden, scale_log2, queue);
+        else
+            hipLaunchKernelGGL((attn_varlen_f32_kernel<kWavesF32, 1>), dim3((unsigned)std::min(items, cus)), block, 0, st,
+                               q, 3 * hidden, o, hidden, cu_seqlens, order, batch, n_heads, hidden, scale_log2, queue);
         TZH_LAUNCHED("attn_varlen_f32_kernel");
         return TZH_OK;
     }

@@ -14,8 +14,8 @@
 // Design:
 //   - Output tiles of 128 x 128, 64 x 128, 64 x 64 or 32 x 32 per 256-thread
 //     block (choose_tile): the large ones reuse each operand most, the small
-//     ones leave fewer CUs idle.  Four waves split the tile, or (32 x 32) the
-//     k steps of a stage, their sums meeting in LDS at the end.
+//     ones leave fewer CUs idle.  Four waves split the tile, or (32 x 32 in
+//     f32) the k steps of a stage, their sums meeting in LDS at the end.
 //   - k runs in stages of 16 to 128, the deeper the smaller the tile, so that
 //     a stage holds about as many matrix instructions (2 048 cycles a wave;
 //     32 x 32: 1 024) as a load takes to arrive.  Operands are loaded into
@@ -67,6 +67,7 @@ struct Tile {
     static constexpr int WM = KW == 1 ? 2 : 1, WN = KW == 1 ? 2 : 1;
     static constexpr int MT = BM / WM / 16, NT = BN / WN / 16;  // 16 x 16 MFMA tiles of a wave
     static_assert(WM * WN * KW == 4 && BK % (16 * KW) == 0, "four waves, whole 16-wide k groups each");
+    static_assert(MT >= 1 && NT >= 1, "whole MFMA tiles");
     static_assert(KW == 1 || MT * NT == KW, "split k: each wave finishes one MFMA tile");
 };
 // LDS pitches in elements: a [row][k] tile's rows start on sixteen different
@@ -366,10 +367,10 @@ struct TileShape {
 };
 constexpr TileShape kTileShapes[] = {{128, 128, 8}, {64, 128, 8}, {64, 64, 7}, {32, 32, 4}};
 
-int choose_tile(int num_cus, int64_t m, int64_t n, int64_t batches, bool split_k) {
+int choose_tile(int num_cus, int64_t m, int64_t n, int64_t batches) {
     int best = 0;
     double best_cost = 0;
-    for (int i = 0; i < (split_k ? 4 : 3); i++) {
+    for (int i = 0; i < 4; i++) {
         const TileShape &t = kTileShapes[i];
         const double tiles = (double)((m + t.bm - 1) / t.bm) * (double)((n + t.bn - 1) / t.bn) * (double)batches;
         const double cost = std::ceil(tiles / num_cus) * t.bm * t.bn / t.rate8;
@@ -415,7 +416,7 @@ int tzh_gemm_fp_launch(hipStream_t st, int num_cus, int32_t dtype, bool a_trans,
         if (op != TZH_OP_ADD && !tzh_ew::unary_ok(op))
             return tzh_fail(TZH_ERR_UNSUPPORTED_OP, "epilogue op %d is not a unary op or a bias add", op);
     }
-    const int ts = choose_tile(num_cus, d.m, d.n, batches, d.split_k);
+    const int ts = choose_tile(num_cus, d.m, d.n, batches);
     const int64_t tm = (d.m + kTileShapes[ts].bm - 1) / kTileShapes[ts].bm;
     const int64_t tn = (d.n + kTileShapes[ts].bn - 1) / kTileShapes[ts].bn;
     if (batches > ((int64_t)1 << 31) / (tm * tn)) return tzh_fail(TZH_ERR_TOO_LARGE, "GEMM grid too large");
@@ -454,7 +455,16 @@ int tzh_gemm_fp_launch(hipStream_t st, int num_cus, int32_t dtype, bool a_trans,
         case 0: launch_tile<T, Tile<T, 128, 128, 16, 1>>(st, a_trans, b_trans, A, B, Y, g, blocks); break;
         case 1: launch_tile<T, Tile<T, 64, 128, 16 * E, 1>>(st, a_trans, b_trans, A, B, Y, g, blocks); break;
         case 2: launch_tile<T, Tile<T, 64, 64, 32 * E, 1>>(st, a_trans, b_trans, A, B, Y, g, blocks); break;
-        default: launch_tile<T, Tile<T, 32, 32, 64 * E, 4>>(st, a_trans, b_trans, A, B, Y, g, blocks); break;
+        default:
+            // split k in f32 only: f64 keeps the one order of its sums
+            if constexpr (sizeof(T) == 4) {
+                if (d.split_k) {
+                    launch_tile<T, Tile<T, 32, 32, 64 * E, 4>>(st, a_trans, b_trans, A, B, Y, g, blocks);
+                    break;
+                }
+            }
+            launch_tile<T, Tile<T, 32, 32, 64 * E, 1>>(st, a_trans, b_trans, A, B, Y, g, blocks);
+            break;
         }
         TZH_LAUNCHED("gemm_mfma_kernel");
         return TZH_OK;

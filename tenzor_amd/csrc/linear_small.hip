@@ -11,7 +11,8 @@
 //   - Blocks of 16 or 32 rows by 64 outputs (four waves, 16 outputs each) or
 //     16 rows by 16 outputs (the four waves share k): enough blocks for the
 //     chip at any size this kernel is used for.
-//   - A block holds its rows' k range (chunks of 512 or 1024) in LDS, split
+//   - A block holds its rows' k range (chunks of 512, 1024 where the waves
+//     share k) in LDS, split
 //     into f16 halves once.  Every load of a chunk - the wave's codes
 //     straight into registers, the rows - is issued before the first wait;
 //     nothing is staged in rounds.
@@ -76,7 +77,7 @@ constexpr int kEUnset = 200;  // row exponent before any value: above every 15 -
 template <typename TX, typename TC, typename TR, int EPI, bool WT, bool SCALED, bool LNP, int BM, int WN, int NF>
 __global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
     constexpr bool SPLIT = sizeof(TX) == 4;
-    constexpr int WK = 4 / WN, KC = BM == 32 ? 512 : 1024, P = KC + 8, MF = BM / 16;
+    constexpr int WK = 4 / WN, KC = WK == 1 ? 512 : 1024, P = KC + 8, MF = BM / 16;
     constexpr int TPR = 256 / BM;             // threads per row
     constexpr int NP = KC / (8 * TPR);        // 8-value pieces per thread per chunk
     constexpr int CS = KC / 64 / WK;          // 64-code groups of a wave per chunk
@@ -124,17 +125,47 @@ __global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
         }
     };
 
-    f32x4_t acc[MF][NF];
+    // A model's linears keep four partial sums, by the 64-code group modulo
+    // four, added in order at the end: the same sums whether one wave holds
+    // all four or four waves one each, so a sequence's embedding does not
+    // depend on the tile, that is on the rest of its batch.
+    constexpr int NQ = WT ? 4 / WK : 1;
+    f32x4_t acc[NQ][MF][NF];
 #pragma unroll
-    for (int f = 0; f < MF; f++)
+    for (int p = 0; p < NQ; p++)
 #pragma unroll
-        for (int h = 0; h < NF; h++) acc[f][h] = f32x4_t{};
+        for (int f = 0; f < MF; f++)
+#pragma unroll
+            for (int h = 0; h < NF; h++) acc[p][f][h] = f32x4_t{};
     int ecur = kEUnset;  // the thread's row's exponent
     int eacc[MF];        // the exponent of acc[f]'s sums
 #pragma unroll
     for (int f = 0; f < MF; f++) eacc[f] = kEUnset;
 
-    // 64-code groups of the chunk at c0, and this wave's: g0 .. g0 + gn - 1
+    // The epilogue's operands, loaded with the first chunk: lane (token r16,
+    // g) of fragments (f, h) holds outputs 4 g + e of 16.  Columns past n
+    // repeat the last one's (never stored).
+    float sc[NF][4], bs[NF][4];
+    TR rv[MF][NF][EPI == SE_RES ? 4 : 1];
+    auto load_epi = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int h = 0; h < NF; h++) {
+            const int n = n0 + 16 * (NF * wn + h) + 4 * g;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int ne = n + e < a.n ? n + e : a.n - 1;
+                sc[h][e] = f16_bits_to_f32(a.scale[ne]);
+                bs[h][e] = a.bias ? a.bias[ne] : 0.0f;
+                if constexpr (EPI == SE_RES)
+#pragma unroll
+                    for (int f = 0; f < MF; f++) {
+                        const int t = t0 + 16 * f + r16 < a.m ? t0 + 16 * f + r16 : a.m - 1;
+                        rv[f][h][e] = ((const TR *)a.res)[(size_t)t * a.n + ne];
+                    }
+            }
+        }
+    };
+    // 64-code groups of the chunk at c0; this wave's are wk, wk + WK, ...
     auto groups_of = [&](int c0) __attribute__((always_inline)) {
         return ((a.k - c0 < KC ? a.k - c0 : KC) + 63) / 64;
     };
@@ -144,52 +175,63 @@ __global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
     } wc, wnext;
     TX xv[NP][8];
     auto load_chunk = [&](int c0, Codes &wd) __attribute__((always_inline)) {
-        const int groups = groups_of(c0), per = (groups + WK - 1) / WK, g0 = wk * per;
-        const int gn = groups - g0 < per ? groups - g0 : per;
+        const int groups = groups_of(c0);
 #pragma unroll
         for (int s = 0; s < CS; s++)
-            if (s < gn)
+            if (WK * s + wk < groups)
 #pragma unroll
-                for (int h = 0; h < NF; h++) wd.v[s][h] = load_codes(nrow[h], c0 + 64 * (g0 + s) + 16 * g);
+                for (int h = 0; h < NF; h++) wd.v[s][h] = load_codes(nrow[h], c0 + 64 * (WK * s + wk) + 16 * g);
 #pragma unroll
         for (int i = 0; i < NP; i++)
             if (8 * TPR * i < 64 * groups) load_row8<TX>(xrow, c0 + 8 * (sub + TPR * i), a.k, xv[i]);
     };
     if constexpr (SPLIT) load_chunk(0, wc);
+    if constexpr (NF == 1) load_epi();  // (with two fragments a wave they would cost the second block of a CU)
     for (int c0 = 0; c0 < a.k; c0 += KC) {
         if constexpr (!SPLIT) load_chunk(c0, wc);
-        const int groups = groups_of(c0), per = (groups + WK - 1) / WK, g0 = wk * per;
-        const int gn = groups - g0 < per ? groups - g0 : per;
+        const int groups = groups_of(c0);
         if constexpr (LNP) {  // one chunk of 384 columns
-            float sum = 0.0f;
+            // gamma and beta, loaded before the statistics where registers allow
+            constexpr bool EARLY = BM == 16;
+            f32x4_t gg[384 / (8 * TPR)][2], bb[384 / (8 * TPR)][2];
+            auto load_ln = [&](int i) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < 384 / (8 * TPR); i++)
-#pragma unroll
-                for (int e = 0; e < 8; e++) sum += (float)xv[i][e];
-#pragma unroll
-            for (int o = TPR / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
-            const float mean = sum / 384.0f;
-            float sq = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 384 / (8 * TPR); i++)
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const float d = (float)xv[i][e] - mean;
-                    sq += d * d;
+                for (int h = 0; h < 2; h++) {
+                    gg[i][h] = *(const f32x4_t *)(a.gamma + 8 * (sub + TPR * i) + 4 * h);
+                    bb[i][h] = *(const f32x4_t *)(a.beta + 8 * (sub + TPR * i) + 4 * h);
                 }
+            };
+            if constexpr (EARLY)
 #pragma unroll
-            for (int o = TPR / 2; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);
+                for (int i = 0; i < 384 / (8 * TPR); i++) load_ln(i);
+            // sums by sixteenths of the row (16 threads, or 8 holding two
+            // each), then over them in one order for both
+            constexpr int HV = 16 / TPR;
+            auto row_sum = [&](auto &&term) __attribute__((always_inline)) {
+                float s[HV] = {};
+#pragma unroll
+                for (int i = 0; i < 384 / (8 * TPR); i++)
+#pragma unroll
+                    for (int e = 0; e < 8; e++) s[i % HV] += term((float)xv[i][e]);
+                float v = HV == 2 ? s[0] + s[HV - 1] : s[0];
+                if constexpr (HV == 1) v += __shfl_xor(v, 8, 64);
+#pragma unroll
+                for (int o = 4; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+                return v;
+            };
+            const float mean = row_sum([](float x) { return x; }) / 384.0f;
+            const float sq = row_sum([&](float x) { return (x - mean) * (x - mean); });
             const float inv_std = 1.0f / sqrtf(sq / 384.0f + a.eps);
 #pragma unroll
             for (int i = 0; i < 384 / (8 * TPR); i++) {
                 const int j = 8 * (sub + TPR * i);
+                if constexpr (!EARLY) load_ln(i);
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
-                    const f32x4_t gg = *(const f32x4_t *)(a.gamma + j + 4 * h), bb = *(const f32x4_t *)(a.beta + j + 4 * h);
                     f32x4_t y;
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
-                        y[e] = (((float)xv[i][4 * h + e] - mean) * inv_std) * gg[e] + bb[e];
+                        y[e] = (((float)xv[i][4 * h + e] - mean) * inv_std) * gg[i][h][e] + bb[i][h][e];
                         xv[i][4 * h + e] = (TX)y[e];
                     }
                     if (blockIdx.x == 0 && t0 + xr < a.m) *(f32x4_t *)(a.xout + (size_t)trow * 384 + j + 4 * h) = y;
@@ -247,13 +289,17 @@ __global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
 #pragma unroll
                     for (int h = 0; h < NF; h++)
 #pragma unroll
-                        for (int q = 0; q < 4; q++) acc[f][h][q] = ldexp_f(acc[f][h][q], e - eacc[f]);
+                        for (int q = 0; q < 4; q++)
+#pragma unroll
+                            for (int p = 0; p < NQ; p++) acc[p][f][h][q] = ldexp_f(acc[p][f][h][q], e - eacc[f]);
                 eacc[f] = e;
             }
 #pragma unroll
         for (int s = 0; s < CS; s++)
-            if (s < gn) {
-                const int kk = 64 * (g0 + s) + 16 * g;
+            if (WK * s + wk < groups) {
+                constexpr int kChunkGroups = KC / 64;
+                static_assert(kChunkGroups % 4 == 0, "a chunk's groups start a new round of partial sums");
+                const int kk = 64 * (WK * s + wk) + 16 * g, p = s % NQ;
 #pragma unroll
                 for (int j = 0; j < 2; j++) {
                     half8_t wf[NF];
@@ -265,12 +311,12 @@ __global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
                         const half8_t xh = *(const half8_t *)(xhi + o);
 #pragma unroll
                         for (int h = 0; h < NF; h++)
-                            acc[f][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[h], xh, acc[f][h], 0, 0, 0);
+                            acc[p][f][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[h], xh, acc[p][f][h], 0, 0, 0);
                         if constexpr (SPLIT) {
                             const half8_t xl = *(const half8_t *)(xlo + o);
 #pragma unroll
                             for (int h = 0; h < NF; h++)
-                                acc[f][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[h], xl, acc[f][h], 0, 0, 0);
+                                acc[p][f][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[h], xl, acc[p][f][h], 0, 0, 0);
                         }
                     }
                 }
@@ -278,52 +324,44 @@ __global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
         if constexpr (SPLIT) wc = wnext;
     }
 
-    // lane (token r16, g) of fragments (f, h): outputs 4 g + e of 16
+    if constexpr (NF > 1) load_epi();
     if constexpr (WK > 1) {
-        part[tid] = acc[0][0];
+        part[tid] = acc[0][0][0];
         __syncthreads();
         if (w > 0) return;
 #pragma unroll
-        for (int k = 1; k < WK; k++) acc[0][0] += part[64 * k + lane];
+        for (int k = 1; k < WK; k++) acc[0][0][0] += part[64 * k + lane];
+    } else {
+#pragma unroll
+        for (int p = 1; p < NQ; p++)
+#pragma unroll
+            for (int f = 0; f < MF; f++)
+#pragma unroll
+                for (int h = 0; h < NF; h++) acc[0][f][h] += acc[p][f][h];
     }
 #pragma unroll
     for (int h = 0; h < NF; h++) {
         const int n = n0 + 16 * (NF * wn + h) + 4 * g;
         if (n >= a.n) continue;
-        float s[4], b[4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int ne = n + e < a.n ? n + e : a.n - 1;
-            s[e] = f16_bits_to_f32(a.scale[ne]);
-            b[e] = a.bias ? a.bias[ne] : 0.0f;
-        }
 #pragma unroll
         for (int f = 0; f < MF; f++) {
             const int t = t0 + 16 * f + r16;
             if (t >= a.m) continue;
-            float v[4];
+            TC o[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                v[e] = (SCALED ? ldexp_f(acc[f][h][e], -eacc[f]) : acc[f][h][e]) * s[e] + b[e];
-                if constexpr (EPI == SE_GELU) v[e] = gelu_fast(v[e]);
+                float v = (SCALED ? ldexp_f(acc[0][f][h][e], -eacc[f]) : acc[0][f][h][e]) * sc[h][e] + bs[h][e];
+                if constexpr (EPI == SE_GELU) v = gelu_fast(v);
+                if constexpr (EPI == SE_RES) v = (float)rv[f][h][e] + v;
+                o[e] = (TC)v;
             }
             TC *const dst = (TC *)a.c + (size_t)t * a.ldc + n;
             if (n + 4 <= a.n) {
-                if constexpr (EPI == SE_RES) {
-                    TR r[4];
-                    __builtin_memcpy(r, (const TR *)a.res + (size_t)t * a.n + n, 4 * sizeof(TR));
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = (float)r[e] + v[e];
-                }
-                TC o[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) o[e] = (TC)v[e];
                 __builtin_memcpy(dst, o, 4 * sizeof(TC));
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; e++)
-                    if (n + e < a.n)
-                        dst[e] = (TC)(EPI == SE_RES ? (float)((const TR *)a.res)[(size_t)t * a.n + n + e] + v[e] : v[e]);
+                    if (n + e < a.n) dst[e] = o[e];
             }
         }
     }
@@ -337,8 +375,11 @@ int launch_small(hipStream_t st, int num_cus, const SmallArgs &a) {
     const int bn = (a.n + 63) / 64;
     const int64_t rows16 = (a.m + 15) / 16, rows32 = (a.m + 31) / 32;
     if (rows16 > 65535) return tzh_fail(TZH_ERR_TOO_LARGE, "internal: %d rows in the small linear", a.m);
-    if (rows32 * ((a.n + 127) / 128) >= num_cus) {
-        hipLaunchKernelGGL((linear_small_kernel<TX, TC, TR, EPI, WT, SCALED, LNP, 32, 4, 2>),
+    // (a model's linears, with four partial sums, would fall to one block a
+    // CU with two fragments a wave)
+    constexpr int NFM = WT ? 1 : 2;
+    if (NFM == 2 && rows32 * ((a.n + 127) / 128) >= num_cus) {
+        hipLaunchKernelGGL((linear_small_kernel<TX, TC, TR, EPI, WT, SCALED, LNP, 32, 4, NFM>),
                            dim3((unsigned)((a.n + 127) / 128), (unsigned)rows32), dim3(256), 0, st, a);
     } else if (rows32 * bn >= num_cus) {
         hipLaunchKernelGGL((linear_small_kernel<TX, TC, TR, EPI, WT, SCALED, LNP, 32, 4, 1>),
@@ -398,4 +439,40 @@ int tzh_linear_small_launch(hipStream_t st, int num_cus, const void *x, int32_t 
     };
     if (x32) return c32 ? typed(0.0f, 0.0f) : typed(0.0f, (_Float16)0);
     return c32 ? typed((_Float16)0, 0.0f) : typed((_Float16)0, (_Float16)0);
+}
+
+// Rows up to which a model layer's linears run one by one on this file's
+// kernel (five launches a layer, each of enough blocks for the chip) rather
+// than on the fused kernels, whose 64-token panels walk all of a layer's
+// weight stages in series (about 55 us a layer from 1 to 1000 rows).  The
+// line moves with the CUs those rows can spread over.  Measured on 256 CUs,
+// fused -> here: the forward of one sequence of 16 293 -> 144 us, of 128
+// 346 -> 172, of 512 493 -> 298; 5 x 128 367 -> 277; the feed-forward block
+// of 128 rows 23 -> 16, 640 31.5 -> 25.7.  Past the lines: 7 x 128 367 ->
+// 332, 8 x 128 369 -> 375; the block of 700 rows 27 -> 32.
+int64_t tzh_small_layer_rows(int num_cus) { return (int64_t)num_cus * 7 / 2; }
+int64_t tzh_small_ffn_rows(int num_cus) { return (int64_t)num_cus * 5 / 2; }
+
+// A model linear over f32 rows inside the split's range (not row-scaled):
+// C = epi(X W^T s + b) with W8T codes, n a multiple of 384 and k of 64, all
+// pointers 16-byte aligned.  epilogue: TZH_EPI_BIAS, TZH_EPI_BIAS_GELU, or
+// TZH_EPI_BIAS_RES_LN for the rows before the LayerNorm (res added).  gamma
+// non-null (k == 384): x holds rows before a LayerNorm, normalised on the
+// way in and stored to xout (which may not overlap x).
+int tzh_linear_small_model_launch(hipStream_t st, int num_cus, const float *x, const float *gamma, const float *beta,
+                                  float eps, float *xout, const void *w, const uint16_t *scale, const float *bias,
+                                  float *c, int64_t m, int64_t k, int64_t n, int32_t epilogue, const float *res) {
+    if (m <= 0 || m > ((int64_t)1 << 20) || k % 64 || n % 384 || (gamma && (k != 384 || !beta || !xout)))
+        return tzh_fail(TZH_ERR_INVALID_ARGS, "internal: bad small linear");
+    SmallArgs a{};
+    a.x = x, a.w = w, a.scale = scale, a.bias = bias, a.c = c, a.res = res;
+    a.gamma = gamma, a.beta = beta, a.xout = xout, a.eps = eps;
+    a.m = (int)m, a.k = (int)k, a.n = (int)n, a.ldc = (int)n;
+    if (epilogue == TZH_EPI_BIAS_RES_LN)
+        return launch_small<float, float, float, SE_RES, true, false, false>(st, num_cus, a);
+    if (epilogue == TZH_EPI_BIAS_GELU)
+        return gamma ? launch_small<float, float, float, SE_GELU, true, false, true>(st, num_cus, a)
+                     : launch_small<float, float, float, SE_GELU, true, false, false>(st, num_cus, a);
+    return gamma ? launch_small<float, float, float, SE_BIAS, true, false, true>(st, num_cus, a)
+                 : launch_small<float, float, float, SE_BIAS, true, false, false>(st, num_cus, a);
 }
