@@ -281,7 +281,8 @@ struct alignas(sizeof(T) * V) RowVec {
 // softmaxRow (softmax.zig:38-137): max, exp(x - max) summed, then
 // exp(x - max) * (1 / sum) stored (recomputed rather than stored and
 // re-read: the same values, one pass less over memory).  One wave per row
-// of the last axis, V consecutive elements per lane and access.
+// of the last axis, V consecutive elements per lane and access: for rows too
+// long for ew_softmax_held_kernel.
 template <typename T, int V>
 __global__ void __launch_bounds__(256) ew_softmax_rows_kernel(const T *__restrict__ x, T *__restrict__ y,
                                                               int64_t rows, int64_t n) {
@@ -315,7 +316,8 @@ __global__ void __launch_bounds__(256) ew_softmax_rows_kernel(const T *__restric
 }
 
 // softmaxAxis general case (softmax.zig:172-213): one thread per
-// (outer, inner) column of a middle or leading axis.
+// (outer, inner) column of a middle or leading axis too long for
+// ew_softmax_cols_held_kernel.
 template <typename T>
 __global__ void __launch_bounds__(256) ew_softmax_cols_kernel(const T *__restrict__ x, T *__restrict__ y,
                                                               int64_t outer, int64_t n, int64_t inner) {
@@ -337,7 +339,8 @@ __global__ void __launch_bounds__(256) ew_softmax_cols_kernel(const T *__restric
 // layerNorm (layernorm.zig:123-185): mean = sum * (1/N), variance = sum of
 // squared deviations * (1/N), 1 / sqrt(variance + eps), then
 // (x - mean) * inv_std * gamma + beta.  One wave per instance, V
-// consecutive elements per lane and access.
+// consecutive elements per lane and access: for instances too long for
+// ew_layernorm_held_kernel.
 template <typename T, int V>
 __global__ void __launch_bounds__(256) ew_layernorm_kernel(const T *__restrict__ x, const T *__restrict__ g,
                                                            const T *__restrict__ b, T *__restrict__ y,
@@ -374,6 +377,161 @@ __global__ void __launch_bounds__(256) ew_layernorm_kernel(const T *__restrict__
         for (int k = 0; k < V; k++) o.v[k] = ((a.v[k] - mean) * inv_std) * gg.v[k] + bb.v[k];
         yr[c] = o;
     }
+}
+
+// f over the 2^lg lanes of a group of a 256-thread (or larger) block, to every
+// lane of it.  smem: one element per wave.
+template <typename T, typename F>
+__device__ __forceinline__ T group_reduce(T v, int lg, T *smem, F f) {
+    for (int o = (lg < 6 ? 1 << lg : 64) >> 1; o > 0; o >>= 1) v = f(v, __shfl_xor(v, o, 64));
+    if (lg > 6) {  // the same for every thread of the block
+        if ((threadIdx.x & 63) == 0) smem[threadIdx.x >> 6] = v;
+        __syncthreads();
+        const int w0 = (threadIdx.x >> lg) << (lg - 6);  // the first wave of the group
+        v = smem[w0];
+        for (int w = 1; w < 1 << (lg - 6); w++) v = f(v, smem[w0 + w]);
+        __syncthreads();
+    }
+    return v;
+}
+
+// f(LO) + ... + f(LO + N - 1), N a power of two, summed by halves: shorter
+// rounding chains than a running sum, so a lane may hold more of a row.
+template <int N, typename T, typename F>
+__device__ __forceinline__ T sum_by_halves(const F &f, int lo) {
+    if constexpr (N == 1) return f(lo);
+    else return sum_by_halves<N / 2, T>(f, lo) + sum_by_halves<N / 2, T>(f, lo + N / 2);
+}
+
+// Softmax and LayerNorm of rows that fit the registers of up to a block: a
+// group of 2^lg lanes per row, NP vectors a lane.  Both are bound by memory:
+// the row is read once, every load of it issued before the first use, and
+// short rows share a wave (one wave a row left half of it idle at 128 f32
+// and kept one load in flight).  Measured, three passes -> here, us: softmax
+// of f32 49152 x 128 18.4 -> 9.3 (5.4 TB/s), 4000 x 4096 44 -> 26; LayerNorm
+// of 65536 x 768 89 -> 69 (5.8 TB/s), 694 x 2694 25 -> 10.
+template <typename T, int V, int NP>
+__global__ void __launch_bounds__(256) ew_softmax_held_kernel(const T *__restrict__ x, T *__restrict__ y, int64_t rows,
+                                                              int n, int lg) {
+    __shared__ T smem[4];
+    const int g = 1 << lg, lane = threadIdx.x & (g - 1), nv = n / V;
+    const int64_t row = ((int64_t)blockIdx.x << (8 - lg)) + (threadIdx.x >> lg);
+    const int end = row < rows ? nv : 0;
+    const RowVec<T, V> *xr = (const RowVec<T, V> *)(x + row * n);
+    RowVec<T, V> *yr = (RowVec<T, V> *)(y + row * n);
+    RowVec<T, V> h[NP];
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+        if (lane + g * i < end) h[i] = xr[lane + g * i];
+    T m = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+        if (lane + g * i < end)
+#pragma unroll
+            for (int k = 0; k < V; k++) m = fmax(m, h[i].v[k]);
+    m = group_reduce(m, lg, smem, [](T a, T b) { return (T)fmax(a, b); });
+    const T s = sum_by_halves<NP, T>([&](int i) {
+        T t = 0;
+        if (lane + g * i < end)
+            t = sum_by_halves<V, T>([&](int k) { return h[i].v[k] = exp_t(h[i].v[k] - m); }, 0);
+        return t;
+    }, 0);
+    const T inv = (T)1 / group_reduce(s, lg, smem, [](T a, T b) { return a + b; });
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+        if (lane + g * i < end) {
+#pragma unroll
+            for (int k = 0; k < V; k++) h[i].v[k] *= inv;
+            yr[lane + g * i] = h[i];
+        }
+}
+
+template <typename T, int V, int NP>
+__global__ void __launch_bounds__(256) ew_layernorm_held_kernel(const T *__restrict__ x, const T *__restrict__ g_,
+                                                                const T *__restrict__ b_, T *__restrict__ y,
+                                                                int64_t rows, int n, int lg, T eps) {
+    __shared__ T smem[4];
+    const int g = 1 << lg, lane = threadIdx.x & (g - 1), nv = n / V;
+    const int64_t row = ((int64_t)blockIdx.x << (8 - lg)) + (threadIdx.x >> lg);
+    const int end = row < rows ? nv : 0;
+    using RV = RowVec<T, V>;
+    const RV *xr = (const RV *)(x + row * n);
+    RV *yr = (RV *)(y + row * n);
+    const T inv_n = (T)1 / (T)n;
+    // few vectors a lane: gamma and beta are loaded with the row, not after
+    // its statistics (20 rows of 384 f32: 10.1 against 11.2 us a call)
+    constexpr bool EARLY = NP <= 4;
+    RV h[NP], gg[EARLY ? NP : 1], bb[EARLY ? NP : 1];
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+        if (lane + g * i < end) {
+            h[i] = xr[lane + g * i];
+            if constexpr (EARLY) gg[i] = ((const RV *)g_)[lane + g * i], bb[i] = ((const RV *)b_)[lane + g * i];
+        }
+    const auto row_sum = [&](auto term) {
+        return group_reduce(sum_by_halves<NP, T>([&](int i) {
+            T t = 0;
+            if (lane + g * i < end) t = sum_by_halves<V, T>([&](int k) { return term(h[i].v[k]); }, 0);
+            return t;
+        }, 0), lg, smem, [](T a, T b) { return a + b; });
+    };
+    const T mean = row_sum([](T v) { return v; }) * inv_n;
+    const T var = row_sum([&](T v) { return (v - mean) * (v - mean); }) * inv_n;
+    const T inv_std = (T)1 / sqrt_t(var + eps);
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+        if (lane + g * i < end) {
+            const int j = EARLY ? i : 0;
+            if constexpr (!EARLY) gg[0] = ((const RV *)g_)[lane + g * i], bb[0] = ((const RV *)b_)[lane + g * i];
+#pragma unroll
+            for (int k = 0; k < V; k++) h[i].v[k] = ((h[i].v[k] - mean) * inv_std) * gg[j].v[k] + bb[j].v[k];
+            yr[lane + g * i] = h[i];
+        }
+}
+
+// Softmax along a middle or leading axis whose columns fit a block's
+// registers: 2^lx columns by B >> lx threads along the axis, NP elements a
+// thread, so x is read once and y written once, in runs of 2^lx elements
+// (one thread a column passed over memory five times; transposing first and
+// after, six).  Measured, us: f32 [60000, 16, 64], one thread a column 250 ->
+// 121 (4.1 TB/s); through transposes f64 [1, 2000, 16] 38 -> 18, f32 [12, 13,
+// 217] 41 -> 8.6.
+template <typename T, int NP, int B>
+__global__ void __launch_bounds__(B) ew_softmax_cols_held_kernel(const T *__restrict__ x, T *__restrict__ y,
+                                                                 int64_t cols, int n, int64_t inner, int lx) {
+    __shared__ T smem[B];
+    const int cx = threadIdx.x & ((1 << lx) - 1), cy = threadIdx.x >> lx, ny = B >> lx;
+    const int64_t col = ((int64_t)blockIdx.x << lx) + cx;
+    const int end = col < cols ? n : 0;
+    const int64_t base = col / inner * n * inner + col % inner;
+    T h[NP];
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+        if (cy + ny * i < end) h[i] = x[base + (int64_t)(cy + ny * i) * inner];
+    auto all = [&](T v, auto f) {  // f over the threads of the column
+        smem[threadIdx.x] = v;
+        __syncthreads();
+        for (int s = ny >> 1; s > 0; s >>= 1) {
+            if (cy < s) smem[threadIdx.x] = v = f(v, smem[threadIdx.x + (s << lx)]);
+            __syncthreads();
+        }
+        v = smem[cx];
+        __syncthreads();
+        return v;
+    };
+    T m = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+        if (cy + ny * i < end) m = fmax(m, h[i]);
+    m = all(m, [](T a, T b) { return (T)fmax(a, b); });
+    T s = 0;
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+        if (cy + ny * i < end) s += h[i] = exp_t(h[i] - m);
+    const T inv = (T)1 / all(s, [](T a, T b) { return a + b; });
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+        if (cy + ny * i < end) y[base + (int64_t)(cy + ny * i) * inner] = h[i] * inv;
 }
 
 // gather (gather.zig:4-39): output row r is table row indices[r]; a row
@@ -1108,6 +1266,7 @@ struct Planner {
             for (int i = 0; i < n.axis; i++) outer *= n.shape[i];
             for (int i = n.axis + 1; i < n.ndim; i++) inner *= n.shape[i];
             if (inner == 1) return softmax_rows<T>((const T *)x, out, outer, len);
+            if (len <= kColsHeldMax) return softmax_cols_held<T>((const T *)x, out, outer * inner, len, inner);
             if (outer * inner >= 65536) {  // enough columns for one thread each
                 hipLaunchKernelGGL((ew_softmax_cols_kernel<T>), dim3((unsigned)((outer * inner + 255) / 256)), dim3(256),
                                    0, ctx->stream, (const T *)x, out, outer, len, inner);
@@ -1136,15 +1295,9 @@ struct Planner {
             const int64_t rows = numel / len;
             // layernorm.zig:15: default_eps is the f32 1e-5, widened for f64
             constexpr int V = 16 / sizeof(T);
-            const dim3 grid((unsigned)((rows + 3) / 4));
             if (len % V == 0 && aligned16(x) && aligned16(g) && aligned16(b) && aligned16(out))
-                hipLaunchKernelGGL((ew_layernorm_kernel<T, V>), grid, dim3(256), 0, ctx->stream, (const T *)x,
-                                   (const T *)g, (const T *)b, out, rows, len, (T)1e-5f);
-            else
-                hipLaunchKernelGGL((ew_layernorm_kernel<T, 1>), grid, dim3(256), 0, ctx->stream, (const T *)x,
-                                   (const T *)g, (const T *)b, out, rows, len, (T)1e-5f);
-            TZH_LAUNCHED("ew_layernorm_kernel");
-            return TZH_OK;
+                return layernorm_rows<T, V>((const T *)x, (const T *)g, (const T *)b, out, rows, len);
+            return layernorm_rows<T, 1>((const T *)x, (const T *)g, (const T *)b, out, rows, len);
         }
         if (n.kind == TZH_NODE_MATMUL) return launch_matmul(idx, nullptr, 0, out);
         if (n.kind == TZH_NODE_GATHER) {
@@ -1168,16 +1321,79 @@ struct Planner {
 
     static bool aligned16(const void *p) { return ((uintptr_t)p % 16) == 0; }
 
+    // Lanes per row of nv vectors held in registers (log2): whole 16-vector
+    // runs along a row, then four vectors a lane, up to a block.
+    static int held_lanes(int64_t nv) {
+        const int lg = log2_ceil(nv > 64 ? (nv + 3) / 4 : (nv < 16 ? nv : 16));
+        return lg > 8 ? 8 : lg;
+    }
+    // Vectors of a row that 256 lanes hold, 16 each (64 VGPRs); longer rows
+    // are read again for each pass.
+    static constexpr int64_t kHeldVecs = 4096;
+
     template <typename T>
     int softmax_rows(const T *x, T *y, int64_t rows, int64_t len) {
         constexpr int V = 16 / sizeof(T);
-        const dim3 grid((unsigned)((rows + 3) / 4));
-        if (len % V == 0 && aligned16(x) && aligned16(y))
-            hipLaunchKernelGGL((ew_softmax_rows_kernel<T, V>), grid, dim3(256), 0, ctx->stream, x, y, rows, len);
+        if (len % V == 0 && aligned16(x) && aligned16(y)) return softmax_rows_by<T, V>(x, y, rows, len);
+        return softmax_rows_by<T, 1>(x, y, rows, len);
+    }
+
+    template <typename T, int V>
+    int softmax_rows_by(const T *x, T *y, int64_t rows, int64_t len) {
+        const int64_t nv = len / V;
+        const int lg = held_lanes(nv);
+        const int64_t held_blocks = (rows + (256 >> lg) - 1) / (256 >> lg);
+        if (nv <= 1024 && held_blocks <= INT32_MAX)
+            hipLaunchKernelGGL((ew_softmax_held_kernel<T, V, 4>), dim3((unsigned)held_blocks), dim3(256), 0, ctx->stream,
+                               x, y, rows, (int)len, lg);
+        else if (nv <= kHeldVecs && held_blocks <= INT32_MAX)
+            hipLaunchKernelGGL((ew_softmax_held_kernel<T, V, 16>), dim3((unsigned)held_blocks), dim3(256), 0,
+                               ctx->stream, x, y, rows, (int)len, lg);
         else
-            hipLaunchKernelGGL((ew_softmax_rows_kernel<T, 1>), grid, dim3(256), 0, ctx->stream, x, y, rows, len);
+            hipLaunchKernelGGL((ew_softmax_rows_kernel<T, V>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0,
+                               ctx->stream, x, y, rows, len);
         TZH_LAUNCHED("ew_softmax_rows_kernel");
         return TZH_OK;
+    }
+
+    template <typename T, int V>
+    int layernorm_rows(const T *x, const T *g, const T *b, T *y, int64_t rows, int64_t len) {
+        const int64_t nv = len / V;
+        const int lg = held_lanes(nv);
+        const int64_t held_blocks = (rows + (256 >> lg) - 1) / (256 >> lg);
+        if (nv <= 1024 && held_blocks <= INT32_MAX)
+            hipLaunchKernelGGL((ew_layernorm_held_kernel<T, V, 4>), dim3((unsigned)held_blocks), dim3(256), 0,
+                               ctx->stream, x, g, b, y, rows, (int)len, lg, (T)1e-5f);
+        else if (nv <= kHeldVecs && held_blocks <= INT32_MAX)
+            hipLaunchKernelGGL((ew_layernorm_held_kernel<T, V, 16>), dim3((unsigned)held_blocks), dim3(256), 0,
+                               ctx->stream, x, g, b, y, rows, (int)len, lg, (T)1e-5f);
+        else
+            hipLaunchKernelGGL((ew_layernorm_kernel<T, V>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, ctx->stream,
+                               x, g, b, y, rows, len, (T)1e-5f);
+        TZH_LAUNCHED("ew_layernorm_kernel");
+        return TZH_OK;
+    }
+
+    // Longest column that 1024 threads hold in runs of 16 columns: 64
+    // threads by 32 elements (64 f32 each spill at that block size).
+    static constexpr int64_t kColsHeldMax = 2048;
+
+    template <typename T>
+    int softmax_cols_held(const T *x, T *y, int64_t cols, int64_t len, int64_t inner) {
+        // the widest runs (16 to 64 columns) whose columns the block holds
+        auto launch = [&](auto kernel, int threads, int np) -> int {
+            int lx = 6;
+            while (lx > 4 && (int64_t)(threads >> lx) * np < len) lx--;
+            const int64_t blocks = (cols + (1 << lx) - 1) >> lx;
+            if (blocks > INT32_MAX) return tzh_fail(TZH_ERR_TOO_LARGE, "softmax of %lld columns", (long long)cols);
+            hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3((unsigned)threads), 0, ctx->stream, x, y, cols,
+                               (int)len, inner, lx);
+            TZH_LAUNCHED("ew_softmax_cols_held_kernel");
+            return TZH_OK;
+        };
+        if (len <= 128) return launch(ew_softmax_cols_held_kernel<T, 8, 256>, 256, 8);
+        if (len <= 512) return launch(ew_softmax_cols_held_kernel<T, 32, 256>, 256, 32);
+        return launch(ew_softmax_cols_held_kernel<T, 32, 1024>, 1024, 32);
     }
 
     // y = x with its axes permuted: output axis i is input axis perm[i]

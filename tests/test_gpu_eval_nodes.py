@@ -57,6 +57,35 @@ def test_nodes_vs_restatement(dt):
     check_close(LayerNormExpr(tx, tg2, tg2, 2), host, dt)
 
 
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("rows,n", [(1, 1), (257, 7), (37, 8), (5, 63), (4, 65), (9, 67), (19, 260), (6, 268), (3, 1025), (5, 1028), (2, 4095),
+                                    (3, 4097), (3, 8192), (2, 8200), (2, 16384), (1, 16388)])
+def test_rows_at_the_held_kernels_edges(dt, rows, n):
+    """Rows held by part of a wave, a wave, several waves and by none (too
+    long), 16-byte and element accesses, a last block that is partly empty.
+    Sums of n terms in any order differ by at most n ulps of their size; the
+    bar is check_close's."""
+    rng = np.random.default_rng(n)
+    x = (rng.standard_normal((rows, n)) * 3).astype(dt)
+    g, b = rng.standard_normal(n).astype(dt), rng.standard_normal(n).astype(dt)
+    tx, tg, tb = leaf(x), leaf(g), leaf(b)
+    host = {id(tx): x, id(tg): g, id(tb): b}
+    check_close(tx.softmax(-1), host, dt)
+    check_close(LayerNormExpr(tx, tg, tb, 1), host, dt)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("outer,n,inner", [(3, 1, 5), (2, 32, 65), (1, 33, 64), (5, 128, 3), (2, 129, 17), (1, 512, 33),
+                                           (2, 513, 9), (1, 2048, 18), (1, 2049, 5), (2, 4096, 3), (1, 4097, 4)])
+def test_columns_at_the_held_kernels_edges(dt, outer, n, inner):
+    """Columns held by 4 to 64 threads, past them by the transposing path;
+    blocks that span outer indices and end past the last column."""
+    x = (np.random.default_rng(n).standard_normal((outer, n, inner)) * 3).astype(dt)
+    x[0, : n // 2, 0] = -np.inf  # masked entries (the last is finite)
+    tx = leaf(x)
+    check_close(tx.softmax(1), {id(tx): x}, dt)
+
+
 @pytest.mark.parametrize("perm", [(1, 0, 2, 3), (0, 2, 1, 3), (3, 2, 1, 0), (0, 1, 2, 3), (2, 0, 3, 1)])
 def test_transpose_bit_exact(perm):
     """Includes the attention pattern [B,S,H,D] -> [B,H,S,D] (executor.zig:505-520)."""
