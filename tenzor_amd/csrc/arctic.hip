@@ -40,7 +40,7 @@ int tzh_linear_codes_launch(hipStream_t st, int num_cus, const void *x, int32_t 
                             const float *gamma, const float *beta, float eps, float *ln_ws, int64_t ln_ws_rows,
                             bool row_scale);
 int tzh_attention_launch(hipStream_t st, int num_cus, unsigned *queue, const void *qkv, void *out, int32_t dtype,
-                         const int *cu_seqlens, const int *order, int batch, int n_heads, int hidden);
+                         const int *cu_seqlens, const int *order, int batch, int max_len, int n_heads, int hidden);
 size_t tzh_mlp_pack_bytes();
 int tzh_mlp_pack_launch(hipStream_t st, const void *w1, const void *w2, void *out);
 int tzh_mlp_fused_launch(hipStream_t st, int num_cus, const float *x, const void *pack, const uint16_t *s1,
@@ -1032,6 +1032,7 @@ int run_forward(tzh_model *m, float *outputs, float *hidden_out, const uint32_t 
     for (int b = 0; b < batch; b++) cu[b + 1] = cu[b] + lengths[b];
     std::iota(order, order + batch, 0);
     std::stable_sort(order, order + batch, [&](int x, int y) { return lengths[x] > lengths[y]; });
+    const int max_len = lengths[order[0]];
     if (!by_arg) {
         TZH_HIP(hipMemcpyAsync(m->meta, m->host_meta, (size_t)(2 * batch + 1) * 4, hipMemcpyHostToDevice, st));
         TZH_HIP(hipEventRecord(m->meta_done, st));
@@ -1070,7 +1071,7 @@ int run_forward(tzh_model *m, float *outputs, float *hidden_out, const uint32_t 
     }
     if (by_arg) {
         // (once, whatever the timing repetitions: it counts clamped ids)
-        const dim3 grid((unsigned)((lengths[order[0]] + 3) / 4), (unsigned)batch);
+        const dim3 grid((unsigned)((max_len + 3) / 4), (unsigned)batch);
         if (act == TZH_F32)
             hipLaunchKernelGGL(embed_ids_ln_kernel<float>, grid, dim3(256), 0, st, ids, ids_stride, batch, arg, m->meta,
                                (uint32_t)m->cfg.vocab_size, m->bad_ids, m->word.ref(), m->pos.ref(), m->type.ref(),
@@ -1138,8 +1139,8 @@ int run_forward(tzh_model *m, float *outputs, float *hidden_out, const uint32_t 
                             : small_linear(m, st, d.qkv, hf, (float *)m->qkv, T, H, 3 * H, TZH_EPI_BIAS, nullptr);
             }));
             TZH_TRY(stage("attention", [&]() {
-                return tzh_attention_launch(st, cus, m->ctx->work_queue, m->qkv, m->attn, act, d_cu, d_order, batch, 12,
-                                            H);
+                return tzh_attention_launch(st, cus, m->ctx->work_queue, m->qkv, m->attn, act, d_cu, d_order, batch,
+                                            max_len, 12, H);
             }));
             TZH_TRY(stage("attn_out_ln", [&]() {
                 return small_linear(m, st, d.o, (const float *)m->attn, h1f, T, H, H, TZH_EPI_BIAS_RES_LN, hf);
@@ -1167,7 +1168,7 @@ int run_forward(tzh_model *m, float *outputs, float *hidden_out, const uint32_t 
         }));
         TZH_TRY(stage("attention", [&]() {
             return tzh_attention_launch(st, m->ctx->num_cus, m->ctx->work_queue, m->qkv, m->attn, act, d_cu, d_order,
-                                        batch, 12, H);
+                                        batch, max_len, 12, H);
         }));
         // the O-projection, its LayerNorm and the feed-forward block as one
         // kernel (mlp.hip) where the layer has both packs: (attn, h) -> h1,

@@ -527,7 +527,7 @@ __global__ void __launch_bounds__(NW * 64) attn_varlen_f32_kernel(const float *_
 // num_cus: the f32 kernel's persistent grid (one workgroup per CU); queue:
 // its work-queue counters (two, zero between launches: tzh_ctx_work_queue).
 int tzh_attention_launch(hipStream_t st, int num_cus, unsigned *queue, const void *qkv, void *out, int32_t dtype,
-                         const int *cu_seqlens, const int *order, int batch, int n_heads, int hidden) {
+                         const int *cu_seqlens, const int *order, int batch, int max_len, int n_heads, int hidden) {
     if (hidden != n_heads * kHeadDim)
         return tzh_fail(TZH_ERR_INVALID_ARGS, "attention kernel needs head_dim 32 (hidden %d, heads %d)", hidden,
                         n_heads);
@@ -542,15 +542,17 @@ int tzh_attention_launch(hipStream_t st, int num_cus, unsigned *queue, const voi
         // block has a CU of its own.  Measured (12 heads, us a call, of which
         // 17 are the entry point's check of the lengths): one sequence of 512
         // 47 -> 31 and two 48 -> 33 (8 parts), ten of 16 to 512 49 -> 40 (2);
-        // of 128 tokens no change.
+        // of 128 tokens no change; nine of at most 68 25.8 -> 26.6 (2), so
+        // only from max_len 129 on.
         const int64_t items = (int64_t)batch * n_heads, cus = std::max(num_cus, 1);
         const dim3 block(kWavesF32 * 64);
         const float *const q = (const float *)qkv;
         float *const o = (float *)out;
-        if (items * 8 <= cus)
+        const bool deal = max_len > 128;
+        if (deal && items * 8 <= cus)
             hipLaunchKernelGGL((attn_varlen_f32_kernel<kWavesF32, 8>), dim3((unsigned)(items * 8)), block, 0, st, q,
                                3 * hidden, o, hidden, cu_seqlens, order, batch, n_heads, hidden, scale_log2, queue);
-        else if (items * 2 <= cus)
+        else if (deal && items * 2 <= cus)
             hipLaunchKernelGGL((attn_varlen_f32_kernel<kWavesF32, 2>), dim3((unsigned)(items * 2)), block, 0, st, q,
                                3 * hidden, o, hidden, cu_seqlens, order, batch, n_heads, hidden, scale_log2, queue);
         else
@@ -580,13 +582,15 @@ extern "C" int tzh_attention_varlen(tzh_ctx *ctx, const void *qkv, void *out, in
     TZH_HIP(hipMemcpyAsync(cu.data(), cu_seqlens, cu.size() * 4, hipMemcpyDeviceToHost, ctx->stream));
     TZH_HIP(hipStreamSynchronize(ctx->stream));
     if (cu[0] < 0) return tzh_fail(TZH_ERR_INVALID_ARGS, "cu_seqlens[0] is negative");
+    int32_t max_len = 0;
     for (int32_t b = 0; b < batch; b++) {
         const int32_t L = cu[(size_t)b + 1] - cu[(size_t)b];
+        max_len = std::max(max_len, L);
         if (L < 1 || L > kMaxKeys)
             return tzh_fail(TZH_ERR_INVALID_ARGS, "sequence %d has length %d (must be 1..%d)", b, L, kMaxKeys);
     }
     unsigned *queue = nullptr;
     TZH_TRY(tzh_ctx_work_queue(ctx, &queue));
-    return tzh_attention_launch(ctx->stream, ctx->num_cus, queue, qkv, out, dtype, cu_seqlens, nullptr, batch, n_heads,
-                                hidden);
+    return tzh_attention_launch(ctx->stream, ctx->num_cus, queue, qkv, out, dtype, cu_seqlens, nullptr, batch, max_len,
+                                n_heads, hidden);
 }
