@@ -183,7 +183,8 @@ __global__ void __launch_bounds__(256) ew_chain_kernel(const EwProgram p, T *__r
 // thread a column or wave a row through the interpreter): mean over the
 // middle axis of f32 [256, 512, 384] 381 -> 37 us (5.4 TB/s); sum((x - y)^2)
 // over rows of [4096, 4096] 267 -> 21 us, over the middle axis of [4, 4096,
-// 4096] 13.2 ms -> 92 us (5.8 TB/s); mean of 64 rows of 100 000 830 -> 8.8.
+// 4096] 13.2 ms -> 92 us (5.8 TB/s); mean of 64 rows of 100 000 830 -> 8.8;
+// of [1000000, 8, 3] over the middle axis 59 -> 26.
 // The interpreter spends about 4 us on one trip of seven nodes, so it cannot
 // feed a reduction whatever its launch shape (1.1 TB/s with these shapes).
 // ------------------------------------------------------------------------
@@ -1146,6 +1147,30 @@ struct Planner {
         return l;
     }
 
+    // HIP takes no launch of 2^32 or more threads: blocks of 256.
+    static constexpr int64_t kMaxBlocks = 0xffffffffu / 256;
+
+    // reduce_cols' tiles over columns of ncv vectors an outer index: whole
+    // waves along a row, narrower where that leaves fewer lanes idle or the
+    // rows are short.  Where these are far more than the chip's blocks, the
+    // columns are numbered through and the tiles widened, to four threads a
+    // column or as many as get four elements each: a block for each of a
+    // million outer indices, with 24 elements, took 1 140 us where 53 do.
+    static void cols_tiles(RedArgs &a, int64_t ncv, int64_t fill) {
+        a.lg = 6;
+        while (a.lg > 4 && (((ncv - 1) >> a.lg) + 1) << a.lg > ncv + ncv / 8) a.lg--;
+        if (ncv < 16) a.lg = log2_ceil(ncv);
+        const int64_t per_outer = ((ncv - 1) >> a.lg) + 1;
+        a.slots = per_outer << a.lg;
+        a.tiles = per_outer * a.outer;
+        if (a.tiles < 2 * fill) return;
+        a.slots = ncv;
+        const auto tiles = [&](int lg) { return ((a.outer * ncv - 1) >> lg) + 1; };
+        while (a.lg < 8 && ((a.lg < 6 && tiles(a.lg + 1) >= fill) || (256 >> a.lg) * 4 > a.rsz || tiles(a.lg) > kMaxBlocks))
+            a.lg++;
+        a.tiles = tiles(a.lg);
+    }
+
     template <typename T, int V>
     int launch_reduce(int32_t idx, T *out) {
         const tzh_node &n = tape[idx];
@@ -1201,18 +1226,12 @@ struct Planner {
             a.part_len = (nv + a.parts - 1) / a.parts;
             blocks = (outer * a.parts + rows_pb - 1) / rows_pb;
         } else {
-            // column vectors per block: 64 (whole waves along a row) unless a
-            // narrower tile leaves fewer lanes idle
-            const int64_t ncv = (inner + V - 1) / V;
-            a.lg = 6;
-            while (a.lg > 4 && (((ncv - 1) >> a.lg) + 1) << a.lg > ncv + ncv / 8) a.lg--;
-            if (ncv < 16) a.lg = log2_ceil(ncv);
-            a.tiles = ((ncv - 1) >> a.lg) + 1;
-            TZH_TRY(split(a.tiles * outer, rsz / (kMinVecs * (256 >> a.lg))));
+            cols_tiles(a, inner / V, fill);
+            TZH_TRY(split(a.tiles, rsz / (kMinVecs * (256 >> a.lg))));
             a.part_len = (rsz + a.parts - 1) / a.parts;
-            blocks = a.tiles * outer * a.parts;
+            blocks = a.tiles * a.parts;
         }
-        if (blocks > INT32_MAX) return tzh_fail(TZH_ERR_TOO_LARGE, "reduction to %lld elements", (long long)outs);
+        if (blocks > kMaxBlocks) return tzh_fail(TZH_ERR_TOO_LARGE, "reduction to %lld elements", (long long)outs);
         a.finish = a.parts == 1;
         T *const dst = a.finish ? out : (T *)ws;
         const dim3 grid((unsigned)blocks);

@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <deque>
+#include <string>
 #include <vector>
 
 #if defined(__has_feature)
@@ -169,7 +170,22 @@ int lane_id() { return cur % 64; }
 int wave_id() { return cur / 64; }
 void *wave_slot(int lane) { return &slots[((size_t)(cur / 64) * 64 + (size_t)lane) * kSlot]; }
 
+// Recording (tzh_emu_record): launches are written down, one line each, and
+// not run, so that the launch shapes of any size can be checked.
+static bool g_recording = false;
+static std::string g_recorded;
+
 void launch(const char *name, dim3 grid, dim3 block, void (*body)(void *), void *ctx) {
+    if (g_recording) {
+        g_recorded += std::string(name) + " " + std::to_string(grid.x) + " " + std::to_string(grid.y) + " " +
+                      std::to_string(grid.z) + " " + std::to_string(block.x) + "\n";
+        return;
+    }
+    // HIP takes no launch of 2^32 or more threads in a dimension
+    if ((unsigned long long)grid.x * block.x >> 32) {
+        std::fprintf(stderr, "EMU: kernel %s launched with %u blocks of %u threads\n", name, grid.x, block.x);
+        std::abort();
+    }
     if (block.y != 1 || block.z != 1 || block.x == 0 || block.x > 1024) {
         std::fprintf(stderr, "EMU: unsupported block shape for %s\n", name);
         std::abort();
@@ -253,6 +269,14 @@ void launch(const char *name, dim3 grid, dim3 block, void (*body)(void *), void 
 }
 
 }  // namespace emu
+
+// on != 0 starts a recording; on == 0 ends it.  Returns the lines
+// "kernel grid.x grid.y grid.z block.x" of the launches since it began.
+extern "C" const char *tzh_emu_record(int on) {
+    emu::g_recording = on != 0;
+    if (on) emu::g_recorded.clear();
+    return emu::g_recorded.c_str();
+}
 
 // ---------------------------------------------------------------------------
 // runtime stubs: "device" memory is host memory with exact-size allocations

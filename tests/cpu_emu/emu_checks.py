@@ -915,7 +915,65 @@ def group_gemm_fp():
             assert rc1 == 0 and rc2 == 0 and np.array_equal(fused, split), dt
 
 
-GROUPS = {"eval": group_eval, "gemm_fp": group_gemm_fp, "gemm": group_gemm, "gemm_ln": group_gemm_ln, "range": group_range,
+class Unbacked:
+    """A leaf of any size without memory: its launches can only be recorded."""
+
+    def __init__(self, shape, dt):
+        self.shape = tuple(shape)
+        self.dtype = type("D", (), {"is_floating_point": True, "__str__": lambda s: "torch." + dt})()
+
+    def is_contiguous(self):
+        return True
+
+    def data_ptr(self):
+        return 1 << 40
+
+
+def launches_of(call):
+    """(kernel, blocks, threads a block) of each launch of call(), recorded, not run."""
+    L.tzh_emu_record.restype = C.c_char_p
+    L.tzh_emu_record(1)
+    try:
+        check(call())
+    finally:
+        lines = L.tzh_emu_record(0).decode().splitlines()
+    out = []
+    for line in lines:
+        name, gx, gy, gz, bx = line.rsplit(" ", 4)
+        # HIP takes no launch of 2^32 or more threads in a dimension
+        assert int(gx) * int(bx) < 1 << 32, line
+        out.append((name, int(gx) * int(gy) * int(gz), int(bx)))
+    assert out
+    return out
+
+
+def eval_launches(expr):
+    nodes, leaves = to_tape(expr)
+    arr = (_abi.Leaf * max(1, len(leaves)))()
+    for i, t in enumerate(leaves):
+        arr[i].data = t.data.data_ptr()
+        arr[i].ndim = len(t.shape)
+        for j, d in enumerate(t.shape):
+            arr[i].shape[j] = d
+    tape = (_abi.Node * len(nodes))(*nodes)
+    return launches_of(lambda: L.tzh_eval_into(CTX, tape, len(nodes), arr, len(leaves),
+                                               _abi.F64 if expr.dtype == "float64" else _abi.F32, 1 << 41))
+
+
+def group_launches():
+    """Launch shapes at sizes that no emulated run reaches."""
+    # reductions along a middle axis: no more threads than elements where the
+    # columns fill the chip, whatever their length and number per outer index
+    for dt in ("float32", "float64"):
+        for shape in [(1000000, 8, 2), (1000000, 8, 3), (300000, 3, 12), (65536, 8, 8), (100000, 2, 100), (1 << 24, 8, 2),
+                      (20000000, 4, 3), (1 << 26, 2, 32), (1 << 29, 1, 2)]:
+            leaf = Tensor(Unbacked(shape, dt))
+            for e in (leaf, leaf.abs()):
+                _, blocks, threads = eval_launches(ReduceExpr("sum", e, (1,)))[0]
+                assert blocks * threads <= shape[0] * shape[1] * shape[2], (shape, blocks)
+
+
+GROUPS = {"launches": group_launches, "eval": group_eval, "gemm_fp": group_gemm_fp, "gemm": group_gemm, "gemm_ln": group_gemm_ln, "range": group_range,
           "attention": group_attention,
           "arctic": group_arctic, "arctic_f16w": group_arctic_f16w, "embed": group_embed, "models": group_models, "mlp": group_mlp,
           "mlp_split": group_mlp_split,

@@ -34,7 +34,7 @@ def emu_env():
     return env
 
 
-GROUPS = ["eval", "attention", "gemm", "gemm_ln", "range", "models", "nodes", "gemm_fp", "mlp", "mlp_split", "arctic",
+GROUPS = ["launches", "eval", "attention", "gemm", "gemm_ln", "range", "models", "nodes", "gemm_fp", "mlp", "mlp_split", "arctic",
           "arctic_f16w"]
 # emulated CU count per group (default 16): two CUs give the fused
 # feed-forward kernel blocks of several panels at a size the emulation

@@ -253,6 +253,25 @@ def test_reduce_launch_shapes(ctx, shape, axis, dtype, chain):
             assert (np.abs(got - ref) <= bound + (0 if not chain else 2 * eps)).all(), (op, off)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("shape", [(300, 8, 3), (513, 2, 2), (70, 3, 8), (33, 9, 12), (5, 33, 70), (17, 16, 64),
+                                   (600, 1, 2), (2100, 5, 4), (9, 40, 4), (65, 17, 6)])
+def test_reduce_short_columns(ctx, shape, dtype):
+    """Tiles of columns that lie in several outer indices, whole vectors and
+    single elements, 256 to 16 columns a block, one leaf and a chain: maxima
+    exact; each side of a sum of n terms is within n rounding errors of its
+    terms' magnitude."""
+    np_dt = np.float32 if dtype == torch.float32 else np.float64
+    x = np.random.default_rng(12).standard_normal(shape).astype(np_dt)
+    leaf = Tensor(torch.from_numpy(x).to(DEV))
+    for e, v in ((leaf, x), (leaf.abs(), np.abs(x))):
+        v = v.astype(np.float64)
+        got = eval(ReduceExpr("reduce_max", e, (1,)), ctx).cpu().numpy()
+        assert (got == v.max(1)).all()
+        got = eval(ReduceExpr("sum", e, (1,)), ctx).cpu().numpy()
+        assert (np.abs(got - v.sum(1)) <= np.finfo(np_dt).eps * shape[1] * np.abs(v).sum(1)).all()
+
+
 def test_reduce_feeds_chain(ctx):
     rng = np.random.default_rng(6)
     x = rng.standard_normal((40, 300)).astype(np.float32)

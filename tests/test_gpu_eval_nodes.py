@@ -86,6 +86,14 @@ def test_columns_at_the_held_kernels_edges(dt, outer, n, inner):
     check_close(tx.softmax(1), {id(tx): x}, dt)
 
 
+def test_reduce_of_more_outer_indices_than_blocks():
+    """2^24 outer indices of two columns: HIP takes fewer than 2^24 blocks of
+    256 threads.  Sums of two elements round once: bit for bit torch's."""
+    x = torch.randn(1 << 24, 2, 2, device="cuda")
+    got = eval(ReduceExpr("sum", Tensor(x), (1,)))
+    assert torch.equal(got, x[:, 0] + x[:, 1])
+
+
 @pytest.mark.parametrize("perm", [(1, 0, 2, 3), (0, 2, 1, 3), (3, 2, 1, 0), (0, 1, 2, 3), (2, 0, 3, 1)])
 def test_transpose_bit_exact(perm):
     """Includes the attention pattern [B,S,H,D] -> [B,H,S,D] (executor.zig:505-520)."""
