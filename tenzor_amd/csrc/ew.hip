@@ -1221,6 +1221,7 @@ struct Planner {
             const int64_t nv = rsz / V;
             a.lg = log2_ceil(nv / 4 > 16 ? nv / 4 : (nv < 16 ? nv : 16));
             if (a.lg > 8) a.lg = 8;
+            while (a.lg > 0 && ((outer - 1) >> (8 - a.lg)) + 1 > kMaxBlocks) a.lg--;
             const int64_t rows_pb = (int64_t)1 << (8 - a.lg);
             TZH_TRY(split((outer + rows_pb - 1) / rows_pb, nv / (kMinVecs << a.lg)));
             a.part_len = (nv + a.parts - 1) / a.parts;
@@ -1290,7 +1291,11 @@ struct Planner {
             for (int i = 0; i < n.axis; i++) outer *= n.shape[i];
             for (int i = n.axis + 1; i < n.ndim; i++) inner *= n.shape[i];
             if (inner == 1) return softmax_rows<T>((const T *)x, out, outer, len);
-            if (len <= kColsHeldMax) return softmax_cols_held<T>((const T *)x, out, outer * inner, len, inner);
+            if (len <= kColsHeldMax) {
+                bool held = false;
+                TZH_TRY(softmax_cols_held<T>((const T *)x, out, outer * inner, len, inner, &held));
+                if (held) return TZH_OK;
+            }
             if (outer * inner >= 65536) {  // enough columns for one thread each
                 hipLaunchKernelGGL((ew_softmax_cols_kernel<T>), dim3((unsigned)((outer * inner + 255) / 256)), dim3(256),
                                    0, ctx->stream, (const T *)x, out, outer, len, inner);
@@ -1367,10 +1372,10 @@ struct Planner {
         const int64_t nv = len / V;
         const int lg = held_lanes(nv);
         const int64_t held_blocks = (rows + (256 >> lg) - 1) / (256 >> lg);
-        if (nv <= 1024 && held_blocks <= INT32_MAX)
+        if (nv <= 1024 && held_blocks <= kMaxBlocks)
             hipLaunchKernelGGL((ew_softmax_held_kernel<T, V, 4>), dim3((unsigned)held_blocks), dim3(256), 0, ctx->stream,
                                x, y, rows, (int)len, lg);
-        else if (nv <= kHeldVecs && held_blocks <= INT32_MAX)
+        else if (nv <= kHeldVecs && held_blocks <= kMaxBlocks)
             hipLaunchKernelGGL((ew_softmax_held_kernel<T, V, 16>), dim3((unsigned)held_blocks), dim3(256), 0,
                                ctx->stream, x, y, rows, (int)len, lg);
         else
@@ -1385,10 +1390,10 @@ struct Planner {
         const int64_t nv = len / V;
         const int lg = held_lanes(nv);
         const int64_t held_blocks = (rows + (256 >> lg) - 1) / (256 >> lg);
-        if (nv <= 1024 && held_blocks <= INT32_MAX)
+        if (nv <= 1024 && held_blocks <= kMaxBlocks)
             hipLaunchKernelGGL((ew_layernorm_held_kernel<T, V, 4>), dim3((unsigned)held_blocks), dim3(256), 0,
                                ctx->stream, x, g, b, y, rows, (int)len, lg, (T)1e-5f);
-        else if (nv <= kHeldVecs && held_blocks <= INT32_MAX)
+        else if (nv <= kHeldVecs && held_blocks <= kMaxBlocks)
             hipLaunchKernelGGL((ew_layernorm_held_kernel<T, V, 16>), dim3((unsigned)held_blocks), dim3(256), 0,
                                ctx->stream, x, g, b, y, rows, (int)len, lg, (T)1e-5f);
         else
@@ -1402,14 +1407,16 @@ struct Planner {
     // threads by 32 elements (64 f32 each spill at that block size).
     static constexpr int64_t kColsHeldMax = 2048;
 
+    // *held = false (nothing launched) past what one launch takes.
     template <typename T>
-    int softmax_cols_held(const T *x, T *y, int64_t cols, int64_t len, int64_t inner) {
+    int softmax_cols_held(const T *x, T *y, int64_t cols, int64_t len, int64_t inner, bool *held) {
         // the widest runs (16 to 64 columns) whose columns the block holds
         auto launch = [&](auto kernel, int threads, int np) -> int {
             int lx = 6;
             while (lx > 4 && (int64_t)(threads >> lx) * np < len) lx--;
             const int64_t blocks = (cols + (1 << lx) - 1) >> lx;
-            if (blocks > INT32_MAX) return tzh_fail(TZH_ERR_TOO_LARGE, "softmax of %lld columns", (long long)cols);
+            *held = blocks <= 0xffffffffu / threads;
+            if (!*held) return TZH_OK;
             hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3((unsigned)threads), 0, ctx->stream, x, y, cols,
                                (int)len, inner, lx);
             TZH_LAUNCHED("ew_softmax_cols_held_kernel");

@@ -374,6 +374,7 @@ int choose_tile(int num_cus, int64_t m, int64_t n, int64_t batches) {
         const TileShape &t = kTileShapes[i];
         const double tiles = (double)((m + t.bm - 1) / t.bm) * (double)((n + t.bn - 1) / t.bn) * (double)batches;
         const double cost = std::ceil(tiles / num_cus) * t.bm * t.bn / t.rate8;
+        if (i > 0 && tiles * kThreads > 4294967295.0) break;  // past what HIP launches
         if (i == 0 || cost < best_cost) best = i, best_cost = cost;
     }
     return best;

@@ -24,7 +24,7 @@ sys.path.insert(0, ROOT)
 
 import oracle  # noqa: E402
 from tenzor_amd import _abi, synth  # noqa: E402
-from tenzor_amd.expr import BinaryExpr, ReduceExpr, ScalarExpr, Tensor, UnaryExpr, to_tape  # noqa: E402
+from tenzor_amd.expr import BinaryExpr, LayerNormExpr, ReduceExpr, ScalarExpr, Tensor, UnaryExpr, to_tape  # noqa: E402
 
 L = _abi.bind(C.CDLL(os.environ.get("TZH_EMU_LIB", os.path.join(HERE, "libtenzor_hip_emu.so"))))
 CTX = C.c_void_p()
@@ -971,6 +971,18 @@ def group_launches():
             for e in (leaf, leaf.abs()):
                 _, blocks, threads = eval_launches(ReduceExpr("sum", e, (1,)))[0]
                 assert blocks * threads <= shape[0] * shape[1] * shape[2], (shape, blocks)
+    # what takes a group of lanes or a block an item: sizes whose widest groups
+    # HIP would refuse (launches_of checks each)
+    for dt in ("float32", "float64"):
+        for rows, n in [(1 << 25, 261), (1 << 24, 1030), ((1 << 26) - 4, 2)]:
+            leaf, g = Tensor(Unbacked((rows, n), dt)), Tensor(Unbacked((n,), dt))
+            eval_launches(ReduceExpr("sum", leaf, (1,)))
+            eval_launches(leaf.softmax(1))
+            eval_launches(LayerNormExpr(leaf, g, g))
+        for shape in [(1 << 29, 2, 2), (1 << 23, 40, 128), (1 << 26, 200, 4)]:
+            eval_launches(Tensor(Unbacked(shape, dt)).softmax(1))
+        for b, m, k, n in [(9 << 20, 40, 4, 20), (9 << 20, 60, 4, 70), ((1 << 24) - 1, 100, 3, 4)]:
+            eval_launches(Tensor(Unbacked((b, m, k), dt)).matmul(Tensor(Unbacked((k, n), dt))))
 
 
 GROUPS = {"launches": group_launches, "eval": group_eval, "gemm_fp": group_gemm_fp, "gemm": group_gemm, "gemm_ln": group_gemm_ln, "range": group_range,
