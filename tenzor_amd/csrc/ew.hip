@@ -318,7 +318,7 @@ __global__ void __launch_bounds__(256) ew_softmax_rows_kernel(const T *__restric
 
 // softmaxAxis general case (softmax.zig:172-213): one thread per
 // (outer, inner) column of a middle or leading axis too long for
-// ew_softmax_cols_held_kernel.
+// ew_softmax_cols_held_kernel, or of one or two elements.
 template <typename T>
 __global__ void __launch_bounds__(256) ew_softmax_cols_kernel(const T *__restrict__ x, T *__restrict__ y,
                                                               int64_t outer, int64_t n, int64_t inner) {
@@ -529,9 +529,13 @@ __global__ void __launch_bounds__(B) ew_softmax_cols_held_kernel(const T *__rest
 #pragma unroll
     for (int i0 = 0; i0 < NP; i0 += 8) {  // by eights: a shorter rounding chain
         T t = 0;
+        if constexpr (NP == 8) {  // a thread may hold a column of eight alone
+            t = sum_by_halves<8, T>([&](int i) { return cy + ny * i < end ? h[i] = exp_t(h[i] - m) : (T)0; }, 0);
+        } else {
 #pragma unroll
-        for (int i = i0; i < i0 + 8; i++)
-            if (cy + ny * i < end) t += h[i] = exp_t(h[i] - m);
+            for (int i = i0; i < i0 + 8; i++)
+                if (cy + ny * i < end) t += h[i] = exp_t(h[i] - m);
+        }
         s += t;
     }
     const T inv = (T)1 / all(s, [](T a, T b) { return a + b; });
@@ -1291,7 +1295,9 @@ struct Planner {
             for (int i = 0; i < n.axis; i++) outer *= n.shape[i];
             for (int i = n.axis + 1; i < n.ndim; i++) inner *= n.shape[i];
             if (inner == 1) return softmax_rows<T>((const T *)x, out, outer, len);
-            if (len <= kColsHeldMax) {
+            // (columns of one or two gain nothing from being held: a thread each
+            // over 4 M of two took 20 us, held 25)
+            if (len <= kColsHeldMax && (len > 2 || outer * inner < 65536)) {
                 bool held = false;
                 TZH_TRY(softmax_cols_held<T>((const T *)x, out, outer * inner, len, inner, &held));
                 if (held) return TZH_OK;
@@ -1410,10 +1416,15 @@ struct Planner {
     // *held = false (nothing launched) past what one launch takes.
     template <typename T>
     int softmax_cols_held(const T *x, T *y, int64_t cols, int64_t len, int64_t inner, bool *held) {
-        // the widest runs (16 to 64 columns) whose columns the block holds
+        // the widest runs (16 to 64 columns) whose columns the block holds;
+        // short columns that fill the chip, up to 256, a thread each at 8
+        // elements (f32 [2000, 8, 512], four threads a column -> here 26 ->
+        // 12 us; one thread, three passes 22.5; [100000, 4, 8] 20 -> 7.7, 9.6)
         auto launch = [&](auto kernel, int threads, int np) -> int {
+            const auto holds = [&](int lx) { return (int64_t)(threads >> lx) * np >= len; };
             int lx = 6;
-            while (lx > 4 && (int64_t)(threads >> lx) * np < len) lx--;
+            while (lx > 4 && !holds(lx)) lx--;
+            while (lx < 8 && holds(lx + 1) && cols >> (lx + 1) >= (int64_t)ctx->num_cus * 4) lx++;
             const int64_t blocks = (cols + (1 << lx) - 1) >> lx;
             *held = blocks <= 0xffffffffu / threads;
             if (!*held) return TZH_OK;

@@ -971,6 +971,10 @@ def group_launches():
             for e in (leaf, leaf.abs()):
                 _, blocks, threads = eval_launches(ReduceExpr("sum", e, (1,)))[0]
                 assert blocks * threads <= shape[0] * shape[1] * shape[2], (shape, blocks)
+        # short columns that fill the chip: a thread each
+        for shape in [(1000, 2, 4096), (1000, 3, 1000), (100000, 4, 8), (2000, 8, 512)]:
+            (_, blocks, threads), = eval_launches(Tensor(Unbacked(shape, dt)).softmax(1))
+            assert blocks * threads <= 1.1 * shape[0] * shape[2], (shape, blocks)
     # what takes a group of lanes or a block an item: sizes whose widest groups
     # HIP would refuse (launches_of checks each)
     for dt in ("float32", "float64"):

@@ -94,6 +94,18 @@ def test_reduce_of_more_outer_indices_than_blocks():
     assert torch.equal(got, x[:, 0] + x[:, 1])
 
 
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("outer,n,inner", [(300, 1, 1000), (1100, 2, 251), (90000, 3, 3), (70, 8, 4001), (33, 9, 8000),
+                                           (520, 16, 257), (300, 17, 1000)])
+def test_short_columns(dt, outer, n, inner):
+    """Columns of up to 8 elements by a thread and of up to 16 by two, where
+    they fill the chip; one column masked but for its last element."""
+    x = (np.random.default_rng(n).standard_normal((outer, n, inner)) * 3).astype(dt)
+    x[0, : n - 1, 0] = -np.inf
+    tx = leaf(x)
+    check_close(tx.softmax(1), {id(tx): x}, dt)
+
+
 @pytest.mark.parametrize("perm", [(1, 0, 2, 3), (0, 2, 1, 3), (3, 2, 1, 0), (0, 1, 2, 3), (2, 0, 3, 1)])
 def test_transpose_bit_exact(perm):
     """Includes the attention pattern [B,S,H,D] -> [B,H,S,D] (executor.zig:505-520)."""
