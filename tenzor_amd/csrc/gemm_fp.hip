@@ -457,10 +457,19 @@ int tzh_gemm_fp_launch(hipStream_t st, int num_cus, int32_t dtype, bool a_trans,
         case 1: launch_tile<T, Tile<T, 64, 128, 16 * E, 1>>(st, a_trans, b_trans, A, B, Y, g, blocks); break;
         case 2: launch_tile<T, Tile<T, 64, 64, 32 * E, 1>>(st, a_trans, b_trans, A, B, Y, g, blocks); break;
         default:
+            // short k: one stage of 32 or 64 and a quarter or half of the LDS,
+            // so eight or four blocks a CU in place of two (f32, us, 128 x 128
+            // tiles / stages of 128 / of 32: 100000 x 8 x 8 16 / 30 / 9, 2000
+            // products of 40 x 8 x 20 23 / 38 / 11)
+            if (d.k <= 32) {
+                launch_tile<T, Tile<T, 32, 32, 32, 1>>(st, a_trans, b_trans, A, B, Y, g, blocks);
+                break;
+            }
             // split k in f32 only: f64 keeps the one order of its sums
             if constexpr (sizeof(T) == 4) {
                 if (d.split_k) {
-                    launch_tile<T, Tile<T, 32, 32, 64 * E, 4>>(st, a_trans, b_trans, A, B, Y, g, blocks);
+                    if (d.k <= 64) launch_tile<T, Tile<T, 32, 32, 64, 4>>(st, a_trans, b_trans, A, B, Y, g, blocks);
+                    else launch_tile<T, Tile<T, 32, 32, 64 * E, 4>>(st, a_trans, b_trans, A, B, Y, g, blocks);
                     break;
                 }
             }

@@ -81,6 +81,24 @@ def test_gemm_tile_shapes(ctx, ta, tb, m, n, k):
     assert bool(((Y.double() - ref).abs() <= mag * (k + 2) * 2.0 ** -24 + 2.0 ** -23 * ref.abs()).all())
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("m,n,k", [(20003, 7, 1), (20003, 7, 31), (20003, 7, 32), (20003, 7, 33), (20003, 7, 64),
+                                   (20003, 7, 65), (33, 31, 32), (33, 31, 33)])
+def test_gemm_short_k(ctx, ta, tb, m, n, k):
+    """32 x 32 tiles with one k stage of 32 or 64, and the next size.  Bound
+    as test_gemm_tile_shapes."""
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    A = torch.randn((k, m) if ta else (m, k), device="cuda", generator=g)
+    B = torch.randn((n, k) if tb else (k, n), device="cuda", generator=g)
+    Y = torch.full((m, n), float("nan"), device="cuda")
+    check(lib().tzh_gemm_f32(ctx.handle, ta, tb, m, n, k, 1.0, A.data_ptr(), A.shape[1], B.data_ptr(), B.shape[1], 0.0,
+                             None, 0, 0, Y.data_ptr()))
+    a64 = (A.t() if ta else A).double().contiguous()
+    b64 = (B.t() if tb else B).double().contiguous()
+    ref, mag = a64 @ b64, a64.abs() @ b64.abs()
+    assert bool(((Y.double() - ref).abs() <= mag * (k + 2) * 2.0 ** -24 + 2.0 ** -23 * ref.abs()).all())
+
+
 def test_gemm_row_pitch_and_unaligned(ctx):
     """Row pitches larger than the row (lda > k) and operands off 16-byte
     boundaries (scalar loads)."""
