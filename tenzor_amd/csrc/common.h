@@ -233,7 +233,12 @@ __device__ __forceinline__ uint32_t split_lo_pair(uint32_t hi2, float a, float b
 #endif
 }
 
-__device__ __forceinline__ void split_f32x8(const f32x4_t &a, const f32x4_t &b, half8_t &hi, half8_t &lo) {
+// UP: the low halves times 2^11 instead, lo = f16(2^11 (x - hi)), from a, b and
+// au, bu = 2^11 a, 2^11 b: |r| <= 2^-36 where x is small.
+template <bool UP>
+__device__ __forceinline__ void split_f32x8_by(const f32x4_t &a, const f32x4_t &b, const f32x4_t &au, const f32x4_t &bu,
+                                               half8_t &hi, half8_t &lo) {
+    constexpr float scale = UP ? 2048.0f : 1.0f;
     uint32_t h[4], l[4];
 #pragma unroll
     for (int i = 0; i < 2; i++) {
@@ -243,8 +248,11 @@ __device__ __forceinline__ void split_f32x8(const f32x4_t &a, const f32x4_t &b, 
 #ifdef TZH_EMULATION
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-        l[i] = split_lo_pair(h[i], a[2 * i], a[2 * i + 1]);
-        l[2 + i] = split_lo_pair(h[2 + i], b[2 * i], b[2 * i + 1]);
+        const half2_t p = __builtin_bit_cast(half2_t, h[i]), q = __builtin_bit_cast(half2_t, h[2 + i]);
+        l[i] = __builtin_bit_cast(uint32_t, half2_t{(_Float16)(au[2 * i] - scale * (float)p[0]),
+                                                    (_Float16)(au[2 * i + 1] - scale * (float)p[1])});
+        l[2 + i] = __builtin_bit_cast(uint32_t, half2_t{(_Float16)(bu[2 * i] - scale * (float)q[0]),
+                                                        (_Float16)(bu[2 * i + 1] - scale * (float)q[1])});
     }
 #else
     // the four pairs in one block, one trailing s_nop (see split_lo_pair).
@@ -262,12 +270,16 @@ __device__ __forceinline__ void split_f32x8(const f32x4_t &a, const f32x4_t &b, 
         "v_fma_mixhi_f16 %3, -%7, %16, %15 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
         "s_nop 1"
         : "=&v"(l[0]), "=&v"(l[1]), "=&v"(l[2]), "=&v"(l[3])
-        : "v"(h[0]), "v"(h[1]), "v"(h[2]), "v"(h[3]), "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b[0]),
-          "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(1.0f));
+        : "v"(h[0]), "v"(h[1]), "v"(h[2]), "v"(h[3]), "v"(au[0]), "v"(au[1]), "v"(au[2]), "v"(au[3]), "v"(bu[0]),
+          "v"(bu[1]), "v"(bu[2]), "v"(bu[3]), "v"(scale));
 #endif
     typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
     hi = __builtin_bit_cast(half8_t, u32x4v{h[0], h[1], h[2], h[3]});
     lo = __builtin_bit_cast(half8_t, u32x4v{l[0], l[1], l[2], l[3]});
+}
+
+__device__ __forceinline__ void split_f32x8(const f32x4_t &a, const f32x4_t &b, half8_t &hi, half8_t &lo) {
+    split_f32x8_by<false>(a, b, a, b, hi, lo);
 }
 
 // f32 -> f16 with round-to-nearest-even (v_cvt_f16_f32 honours the default RNE mode).

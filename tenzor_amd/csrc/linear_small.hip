@@ -22,10 +22,18 @@
 //     LayerNorm before this linear (arctic.zig:716-746, 779-809), normalised
 //     on the way into LDS; the first column of blocks stores them.  A
 //     layer's LayerNorms then need no launch of their own.
-//   - Row scaling (SCALED: f32 rows of any magnitude): each row's largest
-//     magnitude in a chunk chooses the exponent e that puts it in [2^14,
-//     2^15), lowered (and the sums rescaled, exactly) by a later chunk that
-//     holds larger values, as gemm_pipe.hip does by stages.
+//   - Row scaling (SCALED: f32 rows of any magnitude): no value is held in
+//     fewer bits than by gemm_pipe.hip, whose stages of 64 columns (32 in the
+//     LayerNorm linears) each take the exponent that puts the row's largest
+//     magnitude so far in [2^14, 2^15).  Here a chunk takes one exponent, and
+//     the low halves are held 2^11 times as large (the codes they multiply
+//     2^-11 times, exactly), which keeps every bit unless the row grows by
+//     more than 2^11 from the chunk's first stage on.  Such rows go in several
+//     passes over the products: the first stage, zeros in place of the rest,
+//     then the rest likewise.  One exponent a chunk with plain low halves lost
+//     them for small values before large ones (2e-4 of the result) and is
+//     0 to 1.3 us a call faster; an exponent a stage, the sums rescaled
+//     between the products, took 60 us at 1000 x 1536 x 1536, this 34.
 #include <type_traits>
 
 #include "pipe.h"
@@ -54,36 +62,36 @@ inline int frexp_exp(float x) {
     return e;
 }
 inline float ldexp_f(float x, int e) { return std::ldexp(x, e); }
+inline int here(int x) { return x; }
 #else
 __device__ __forceinline__ int frexp_exp(float x) { return __builtin_amdgcn_frexp_expf(x); }
 __device__ __forceinline__ float ldexp_f(float x, int e) { return __builtin_amdgcn_ldexpf(x, e); }
-#endif
-
-// Eight consecutive values of a row from column j; columns >= k are 0.
-template <typename TX>
-__device__ __forceinline__ void load_row8(const TX *row, int j, int k, TX (&v)[8]) {
-    if (j + 8 <= k) {
-        __builtin_memcpy(v, row + j, 8 * sizeof(TX));  // (16-byte loads; element alignment is enough)
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; i++) v[i] = j + i < k ? row[j + i] : (TX)0;
-    }
+// x, and what is computed from it, formed anew at each use in a loop instead
+// of held in registers across it
+__device__ __forceinline__ int here(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
 }
+#endif
 
 constexpr int kEUnset = 200;  // row exponent before any value: above every 15 - frexp_exp
 
 // BM rows by 16 NF WN outputs per block (NF fragments of 16 a wave), 4 / WN
 // waves over each chunk's k.
 template <typename TX, typename TC, typename TR, int EPI, bool WT, bool SCALED, bool LNP, int BM, int WN, int NF>
-__global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
+__global__ void __launch_bounds__(256, BM == 16 && WN == 4 && SCALED ? 3 : 2) linear_small_kernel(const SmallArgs a) {
     constexpr bool SPLIT = sizeof(TX) == 4;
     constexpr int WK = 4 / WN, KC = WK == 1 ? 512 : 1024, P = KC + 8, MF = BM / 16;
     constexpr int TPR = 256 / BM;             // threads per row
     constexpr int NP = KC / (8 * TPR);        // 8-value pieces per thread per chunk
     constexpr int CS = KC / 64 / WK;          // 64-code groups of a wave per chunk
     static_assert(WK == 1 || (MF == 1 && NF == 1), "shared k: one fragment to add up");
+    constexpr int GC = EPI == SE_RES ? 32 : 64, GP = 8 * TPR / GC;  // SCALED: columns of a stage, stages of a piece
     __shared__ __attribute__((aligned(16))) _Float16 xs[(SPLIT ? 2 : 1) * BM * P];
-    __shared__ int erow[SCALED ? BM : 1];
+    // SCALED, by row (in LDS for the registers they would hold over the
+    // products): the exponents of this pass and the one before in turns, the
+    // first stage of the chunk that is not done, whether any is left
+    __shared__ int erow[2][SCALED ? BM : 1], pos_row[SCALED ? BM : 1], left_row[SCALED ? BM : 1];
     __shared__ __attribute__((aligned(16))) f32x4_t part[WK > 1 ? 256 : 1];
     _Float16 *const xhi = xs, *const xlo = xs + (SPLIT ? BM * P : 0);
 
@@ -91,29 +99,32 @@ __global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
     const int wn = WK == 1 ? w : 0, wk = WK == 1 ? 0 : w;
     const int t0 = (int)blockIdx.y * BM, n0 = (int)blockIdx.x * (16 * NF * WN);
     const int r16 = lane & 15, g = lane >> 4;
-    // this thread's row of X (clamped: rows past m repeat the last) and
-    // this lane's weight rows (past n: the last)
+    // this thread's row of X (clamped) and this lane's weight rows (past n:
+    // the last)
     const int xr = tid / TPR, sub = tid % TPR;
     const int trow = t0 + xr < a.m ? t0 + xr : a.m - 1;
-    const TX *const xrow = (const TX *)a.x + (size_t)trow * a.k;
-    int nrow[NF];
-#pragma unroll
-    for (int h = 0; h < NF; h++) {
-        const int nr = n0 + 16 * (NF * wn + h) + r16;
-        nrow[h] = nr < a.n ? nr : a.n - 1;
-    }
+    auto nrow = [&](int h) __attribute__((always_inline)) {
+        const int nr = n0 + 16 * (NF * wn + h) + ((SCALED ? here(lane) : lane) & 15);
+        return nr < a.n ? nr : a.n - 1;
+    };
 
-    // codes k .. k + 15 of the lane's weight row, biased (u = q + 128).
-    // Codes at or past k multiply zeros; the loads stay inside the matrix.
-    auto load_codes = [&](int nrow, int k) __attribute__((always_inline)) {
-        typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+    // whether loads past the end of a row of this block may leave the matrix
+    const bool last_rows = !WT && ((int64_t)(n0 + 16 * NF * WN < a.n ? n0 + 16 * NF * WN - 1 : a.n - 1) * a.k +
+                                   (a.k + 63) / 64 * 64) > (int64_t)a.n * a.k;
+    // codes k .. k + 15, k = k64 + 16 g, of the lane's weight row, as they are
+    // stored.  Codes at or past a.k multiply zeros; the loads stay inside the
+    // matrix.  The branch is the block's, so that the loads of a chunk are
+    // issued without a wait between them.
+    auto load_codes = [&](int nrow, int k64) __attribute__((always_inline)) {
+        const int k = k64 + 16 * g;
         if constexpr (WT) {
             const size_t o = (((size_t)(nrow / 384) * (a.k / 64) + k / 64) * 384 + nrow % 384) * 64 + k % 64;
             return *(const u32x4_t *)((const uint8_t *)a.w + o);
         } else {
             const uint8_t *const src = (const uint8_t *)a.w + (size_t)nrow * a.k + k;
-            u32x4_t v = {};
-            if ((size_t)nrow * a.k + k + 16 <= (size_t)a.n * a.k) {
+            u32x4_t v;
+            if (!last_rows || k64 + 64 <= a.k) {
                 __builtin_memcpy(&v, src, 16);
             } else {
                 uint8_t b[16];
@@ -121,7 +132,7 @@ __global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
                 for (int i = 0; i < 16; i++) b[i] = k + i < a.k ? src[i] : (uint8_t)0;
                 __builtin_memcpy(&v, b, 16);
             }
-            return v ^ u32x4_t{0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};
+            return v;
         }
     };
 
@@ -137,10 +148,12 @@ __global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
         for (int f = 0; f < MF; f++)
 #pragma unroll
             for (int h = 0; h < NF; h++) acc[p][f][h] = f32x4_t{};
-    int ecur = kEUnset;  // the thread's row's exponent
-    int eacc[MF];        // the exponent of acc[f]'s sums
-#pragma unroll
-    for (int f = 0; f < MF; f++) eacc[f] = kEUnset;
+    if (SCALED && sub == 0) {
+        erow[1][xr] = kEUnset;
+        pos_row[xr] = 0;
+    }
+    wave_lds_order();  // (a row's threads are of one wave)
+    int turn = 0;
 
     // The epilogue's operands, loaded with the first chunk: lane (token r16,
     // g) of fragments (f, h) holds outputs 4 g + e of 16.  Columns past n
@@ -169,7 +182,6 @@ __global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
     auto groups_of = [&](int c0) __attribute__((always_inline)) {
         return ((a.k - c0 < KC ? a.k - c0 : KC) + 63) / 64;
     };
-    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
     struct Codes {
         u32x4_t v[CS][NF];
     } wc, wnext;
@@ -180,16 +192,38 @@ __global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
         for (int s = 0; s < CS; s++)
             if (WK * s + wk < groups)
 #pragma unroll
-                for (int h = 0; h < NF; h++) wd.v[s][h] = load_codes(nrow[h], c0 + 64 * (WK * s + wk) + 16 * g);
+                for (int h = 0; h < NF; h++) wd.v[s][h] = load_codes(nrow(h), c0 + 64 * (WK * s + wk));
+        const int tl = SCALED ? here(tid) : tid;
+        const int tr = t0 + tl / TPR < a.m ? t0 + tl / TPR : a.m - 1;  // (rows past m repeat the last)
+        const TX *const row = (const TX *)a.x + (size_t)tr * a.k;
 #pragma unroll
         for (int i = 0; i < NP; i++)
-            if (8 * TPR * i < 64 * groups) load_row8<TX>(xrow, c0 + 8 * (sub + TPR * i), a.k, xv[i]);
+            if (8 * TPR * i < 64 * groups) {
+                const int j = c0 + 8 * (tl % TPR + TPR * i);
+                if (c0 + 8 * TPR * (i + 1) <= a.k) {
+                    __builtin_memcpy(xv[i], row + j, 8 * sizeof(TX));  // (16-byte loads; element alignment is enough)
+                } else {  // the row's last piece: what lies past it is cleared where it is used
+#pragma unroll
+                    for (int e = 0; e < 8; e++) xv[i][e] = row[j + e < a.k ? j + e : a.k - 1];
+                }
+            }
     };
+    bool begin = true;
     if constexpr (SPLIT) load_chunk(0, wc);
-    if constexpr (NF == 1) load_epi();  // (with two fragments a wave they would cost the second block of a CU)
-    for (int c0 = 0; c0 < a.k; c0 += KC) {
+    // (with two fragments a wave they would cost the second block of a CU,
+    // with a residual beside the row exponents at 16 x 64 the third)
+    constexpr bool EPI_FIRST = NF == 1 && !(SCALED && EPI == SE_RES && BM == 16 && WN == 4);
+    if constexpr (EPI_FIRST) load_epi();
+    for (int c0 = 0, next; c0 < a.k; c0 = next) {
+        next = c0 + KC;
         if constexpr (!SPLIT) load_chunk(c0, wc);
         const int groups = groups_of(c0);
+#pragma unroll
+        for (int i = 0; i < NP; i++)
+            if (8 * TPR * i < 64 * groups && c0 + 8 * TPR * (i + 1) > a.k)
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    if (c0 + 8 * (sub + TPR * i) + e >= a.k) xv[i][e] = (TX)0;
         if constexpr (LNP) {  // one chunk of 384 columns
             // gamma and beta, loaded before the statistics where registers allow
             constexpr bool EARLY = BM == 16;
@@ -238,34 +272,86 @@ __global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
                 }
             }
         }
+        const int tv = SCALED ? here(tid) : tid, xr = tv / TPR, sub = tv % TPR;
+        int ex = 0, take = KC / GC;  // this pass's exponent and stages of the row
+        int mine = 0, left = 0;      // the stage of this lane's part of piece 0, from the first that is not done
         if constexpr (SCALED) {
-            float mx = 0.0f;
+            const int pos = pos_row[xr];
+            mine = 8 * sub / GC - pos;
+            float at = 0.0f, rest = 0.0f;  // largest magnitudes of stage pos, and from it on
 #pragma unroll
             for (int i = 0; i < NP; i++)
-                if (8 * TPR * i < 64 * groups)
+                if (8 * TPR * i < 64 * groups) {
+                    float mx = 0.0f;
 #pragma unroll
                     for (int e = 0; e < 8; e++) mx = fmaxf(mx, fabsf((float)xv[i][e]));
+                    const int st = mine + i * GP;  // of this lane's part, from pos
+                    at = st == 0 ? mx : at;
+                    rest = st >= 0 ? fmaxf(rest, mx) : rest;
+                }
+            auto over_row = [&](float mx) __attribute__((always_inline)) {
+                mx = fmaxf(mx, dpp_f32<0xB1>(mx));   // lane ^ 1
+                mx = fmaxf(mx, dpp_f32<0x4E>(mx));   // lane ^ 2
+                mx = fmaxf(mx, dpp_f32<0x141>(mx));  // the other quad of the eight
+                if constexpr (TPR == 16) mx = fmaxf(mx, dpp_f32<0x140>(mx));  // the other eight of the sixteen
+                return mx;
+            };
+            at = over_row(at);
+            rest = over_row(rest);
+            // the exponent that puts mx in [2^14, 2^15); zero, inf and NaN have none
+            auto want = [&](float mx) __attribute__((always_inline)) {
+                return mx > 0.0f && mx < INFINITY ? 15 - frexp_exp(mx) : kEUnset;
+            };
+            int e_first = min(erow[turn ^ 1][xr], want(at));
+            const int e_all = min(e_first, want(rest));
+            ex = e_first;
+            if (__any(e_first == kEUnset && e_all < kEUnset)) {
+                // rows that start with a stage of zeros: none of theirs asks
+                // for more than the smallest of the lanes' eights
+                float least = -INFINITY;
 #pragma unroll
-            for (int o = TPR / 2; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-            if (mx > 0.0f) {
-                const int want = 15 - frexp_exp(mx);  // mx 2^want in [2^14, 2^15)
-                ecur = want < ecur ? want : ecur;
+                for (int i = 0; i < NP; i++)
+                    if (8 * TPR * i < 64 * groups) {
+                        float mx = 0.0f;
+#pragma unroll
+                        for (int e = 0; e < 8; e++) mx = fmaxf(mx, fabsf((float)xv[i][e]));
+                        if (mx > 0.0f) least = fmaxf(least, -mx);
+                    }
+                e_first = min(e_first, want(-over_row(least)));
             }
+            const bool whole = e_all == kEUnset || (e_first < kEUnset && e_all >= e_first - 11);
+            ex = whole ? e_all : ex;
+            take = whole ? KC / GC : 1;
+            left = pos + take < 64 * groups / GC;
+            wave_lds_order();
+            if (sub == 0) pos_row[xr] = pos + take;
         }
-        if (c0 > 0) __syncthreads();  // the last chunk's reads are done
+        if (!begin) __syncthreads();  // the last products' reads are done
+        begin = false;
 #pragma unroll
         for (int i = 0; i < NP; i++)
             if (8 * TPR * i < 64 * groups) {
                 const int o = xr * P + 8 * (sub + TPR * i);
                 if constexpr (SPLIT) {
                     f32x4_t lo4, hi4;
+                    const int es = (unsigned)(mine + i * GP) < (unsigned)take ? ex : -1000;  // (others: zeros)
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
-                        lo4[e] = SCALED ? ldexp_f((float)xv[i][e], ecur) : (float)xv[i][e];
-                        hi4[e] = SCALED ? ldexp_f((float)xv[i][4 + e], ecur) : (float)xv[i][4 + e];
+                        lo4[e] = SCALED ? ldexp_f((float)xv[i][e], es) : (float)xv[i][e];
+                        hi4[e] = SCALED ? ldexp_f((float)xv[i][4 + e], es) : (float)xv[i][4 + e];
                     }
                     half8_t h, l;
-                    split_f32x8(lo4, hi4, h, l);
+                    if constexpr (SCALED) {
+                        f32x4_t lou, hiu;
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            lou[e] = 2048.0f * lo4[e];
+                            hiu[e] = 2048.0f * hi4[e];
+                        }
+                        split_f32x8_by<true>(lo4, hi4, lou, hiu, h, l);
+                    } else {
+                        split_f32x8(lo4, hi4, h, l);
+                    }
                     *(half8_t *)(xhi + o) = h;
                     *(half8_t *)(xlo + o) = l;
                 } else {
@@ -275,25 +361,29 @@ __global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
                 }
             }
         if constexpr (SCALED)
-            if (sub == 0) erow[xr] = ecur;
+            if (sub == 0) erow[turn][xr] = ex, left_row[xr] = left;
         __syncthreads();
+        if constexpr (SCALED) {
+            if (__any(left_row[lane % BM])) next = c0;  // the same chunk again
+            else if (sub == 0) pos_row[xr] = 0;
+        }
         // f32: the next chunk's loads fly during this one's products (5 % at
         // k = 1536; with f16 rows, at four blocks a CU, 5 % slower)
         if constexpr (SPLIT)
-            if (c0 + KC < a.k) load_chunk(c0 + KC, wnext);
-        if constexpr (SCALED)
+            if (next < a.k) load_chunk(next, wnext);
+        if constexpr (SCALED) {  // the sums so far, to this pass's exponents
 #pragma unroll
             for (int f = 0; f < MF; f++) {
-                const int e = erow[16 * f + r16];
-                if (e != eacc[f])
+                const int d = erow[turn][16 * f + r16] - erow[turn ^ 1][16 * f + r16];
 #pragma unroll
-                    for (int h = 0; h < NF; h++)
+                for (int h = 0; h < NF; h++)
 #pragma unroll
-                        for (int q = 0; q < 4; q++)
+                    for (int q = 0; q < 4; q++)
 #pragma unroll
-                            for (int p = 0; p < NQ; p++) acc[p][f][h][q] = ldexp_f(acc[p][f][h][q], e - eacc[f]);
-                eacc[f] = e;
+                        for (int p = 0; p < NQ; p++) acc[p][f][h][q] = ldexp_f(acc[p][f][h][q], d);
             }
+            turn ^= 1;
+        }
 #pragma unroll
         for (int s = 0; s < CS; s++)
             if (WK * s + wk < groups) {
@@ -304,19 +394,29 @@ __global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
                 for (int j = 0; j < 2; j++) {
                     half8_t wf[NF];
 #pragma unroll
-                    for (int h = 0; h < NF; h++) wf[h] = codes_to_f16(wc.v[s][h][2 * j], wc.v[s][h][2 * j + 1]);
-#pragma unroll
-                    for (int f = 0; f < MF; f++) {
-                        const int o = (16 * f + r16) * P + kk + 8 * j;
-                        const half8_t xh = *(const half8_t *)(xhi + o);
+                    for (int h = 0; h < NF; h++) {
+                        constexpr uint32_t bias = WT ? 0 : 0x80808080u;  // u = q + 128
+                        wf[h] = codes_to_f16(wc.v[s][h][2 * j] ^ bias, wc.v[s][h][2 * j + 1] ^ bias);
+                    }
+                    auto products = [&](const _Float16 *x, int f, const half8_t (&w)[NF]) __attribute__((always_inline)) {
+                        const half8_t xf = *(const half8_t *)(x + (16 * f + r16) * P + kk + 8 * j);
 #pragma unroll
                         for (int h = 0; h < NF; h++)
-                            acc[p][f][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[h], xh, acc[p][f][h], 0, 0, 0);
-                        if constexpr (SPLIT) {
-                            const half8_t xl = *(const half8_t *)(xlo + o);
+                            acc[p][f][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[h], xf, acc[p][f][h], 0, 0, 0);
+                    };
+                    if constexpr (SCALED) {  // the low halves' codes 2^-11 times, exactly
+                        constexpr _Float16 down = (_Float16)0.00048828125f;
 #pragma unroll
-                            for (int h = 0; h < NF; h++)
-                                acc[p][f][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[h], xl, acc[p][f][h], 0, 0, 0);
+                        for (int f = 0; f < MF; f++) products(xhi, f, wf);
+#pragma unroll
+                        for (int h = 0; h < NF; h++) wf[h] *= down;
+#pragma unroll
+                        for (int f = 0; f < MF; f++) products(xlo, f, wf);
+                    } else {
+#pragma unroll
+                        for (int f = 0; f < MF; f++) {
+                            products(xhi, f, wf);
+                            if constexpr (SPLIT) products(xlo, f, wf);
                         }
                     }
                 }
@@ -324,7 +424,7 @@ __global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
         if constexpr (SPLIT) wc = wnext;
     }
 
-    if constexpr (NF > 1) load_epi();
+    if constexpr (!EPI_FIRST) load_epi();
     if constexpr (WK > 1) {
         part[tid] = acc[0][0][0];
         __syncthreads();
@@ -350,7 +450,8 @@ __global__ void __launch_bounds__(256) linear_small_kernel(const SmallArgs a) {
             TC o[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                float v = (SCALED ? ldexp_f(acc[0][f][h][e], -eacc[f]) : acc[0][f][h][e]) * sc[h][e] + bs[h][e];
+                float v = (SCALED ? ldexp_f(acc[0][f][h][e], -erow[turn ^ 1][16 * f + r16]) : acc[0][f][h][e]) * sc[h][e] +
+                          bs[h][e];
                 if constexpr (EPI == SE_GELU) v = gelu_fast(v);
                 if constexpr (EPI == SE_RES) v = (float)rv[f][h][e] + v;
                 o[e] = (TC)v;

@@ -399,6 +399,29 @@ def group_range():
     cg = linear(a, q, s, bias, np.float32, _abi.EPI_BIAS_GELU)
     assert np.isfinite(cg).all()
     assert (np.abs(cg - g) <= 1.13 * 2.0 ** -21 * (mag + np.abs(exact)) + 2.0 ** -20 * np.abs(g) + 1e-37).all()
+    # few rows whose small values come before a much larger one that weighs
+    # nothing (its codes are 0): the small ones keep both halves up to its
+    # group of 64 columns, 32 with the LayerNorm epilogue
+    rng = np.random.default_rng(37)
+    for m, k, first, big, epi in [(4, 512, 64, 300, _abi.EPI_BIAS), (3, 1600, 1024, 1100, _abi.EPI_BIAS_GELU),
+                                  (40, 640, 64, 127, _abi.EPI_BIAS), (5, 384, 32, 40, _abi.EPI_BIAS_RES_LN)]:
+        a = np.zeros((m, k), np.float32)
+        a[:, :first] = rng.standard_normal((m, first)) * 1e-8
+        a[:, big] = 3.0
+        q = rng.integers(-127, 128, (384, k)).astype(np.int8)
+        q[:, big] = 0
+        s = range_problem(38, 1, k, 384, 1.0)[2]
+        ln = epi == _abi.EPI_BIAS_RES_LN
+        c = linear(a, q, s, None, np.float32, epi, *((np.zeros((m, 384), np.float32), np.ones(384, np.float32),
+                                                      np.zeros(384, np.float32)) if ln else ()))
+        y = (a.astype(np.float64) @ q.astype(np.float64).T) * s.view(np.float16).astype(np.float64)
+        if epi == _abi.EPI_BIAS_GELU:
+            y = 0.5 * y * (1 + np.tanh(0.7978845608 * (y + 0.044715 * y ** 3)))
+        if ln:
+            y = (y - y.mean(1, keepdims=True)) / np.sqrt(y.var(1, keepdims=True) + 1e-12)
+        err = np.linalg.norm(c - y) / np.linalg.norm(y)
+        print(f"  small values first, m={m} k={k}: {err:.2e}", flush=True)
+        assert err < 1e-6, (m, k, err)
     # rows whose scale changes along k (the row exponent drops at a later
     # stage, with the sums so far rescaled), rows that start with zeros, and
     # every epilogue

@@ -179,6 +179,13 @@ inline T __shfl_xor(T v, int mask, int width = 64) {
     return r;
 }
 
+// over the 64 lanes of a whole wave
+inline int __any(int p) {
+    p = p != 0;
+    for (int m = 32; m > 0; m >>= 1) p |= __shfl_xor(p, m, 64);
+    return p;
+}
+
 template <typename T>
 inline T __shfl(T v, int src_lane, int width = 64) {
     static_assert(sizeof(T) <= 256, "slot too small");

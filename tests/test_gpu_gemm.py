@@ -405,3 +405,32 @@ def test_few_row_linear(ctx, m, k, n, epi, dtype):
     # about 2 d / std (their mean and deviation move with them), times gamma
     bar = 1.5 * (2 * tol.max(1, keepdims=True) / std + 2.0 ** -20 * (1 + np.abs(ref))) + half * np.abs(ref) + 2.0 ** -24
     assert (np.abs(got - ref) <= bar).all()
+
+
+@pytest.mark.parametrize("m,k,first,big,epi", [
+    (4, 512, 64, 300, _abi.EPI_BIAS), (3, 1600, 1024, 1100, _abi.EPI_BIAS_GELU), (300, 640, 64, 127, _abi.EPI_BIAS),
+    (1501, 385, 128, 128, _abi.EPI_BIAS), (1030, 448, 64, 447, _abi.EPI_BIAS_GELU),
+    (5, 384, 32, 40, _abi.EPI_BIAS_RES_LN), (300, 384, 32, 63, _abi.EPI_BIAS_RES_LN)])
+def test_few_row_linear_small_values_first(ctx, m, k, first, big, epi):
+    """Rows whose small values come before a much larger one that weighs
+    nothing (its codes are 0): the small ones keep both halves of the split up
+    to its group of 64 columns (32 with the LayerNorm epilogue), so the sums
+    of `first` terms hold to f32's rounding (1e-6 of their norm; in one
+    half alone the error is 2e-4)."""
+    rng = np.random.default_rng(k + m)
+    a = np.zeros((m, k), np.float32)
+    a[:, :first] = rng.standard_normal((m, first)) * 1e-8
+    a[:, big] = 3.0
+    _, q, s, _ = make_problem(3, 1, k, 384)
+    q[:, big] = 0
+    A, Q, S = dev(a), dev(q), dev(s.view(np.int16))
+    z, one = torch.zeros(m, 384, device="cuda"), torch.ones(384, device="cuda")
+    out = torch.empty(m, 384, device="cuda")
+    check(lib().tzh_linear_w8(ctx.handle, A.data_ptr(), _abi.F32, Q.data_ptr(), S.data_ptr(), None, out.data_ptr(), _abi.F32,
+                              m, k, 384, epi, z.data_ptr(), _abi.F32, one.data_ptr(), z.data_ptr(), 1e-12))
+    y = (a.astype(np.float64) @ q.astype(np.float64).T) * s.view(np.float16).astype(np.float64)
+    if epi == _abi.EPI_BIAS_GELU:
+        y = 0.5 * y * (1 + np.tanh(0.7978845608 * (y + 0.044715 * y ** 3)))
+    if epi == _abi.EPI_BIAS_RES_LN:
+        y = (y - y.mean(1, keepdims=True)) / np.sqrt(y.var(1, keepdims=True) + 1e-12)
+    assert np.linalg.norm(out.cpu().numpy() - y) < 1e-6 * np.linalg.norm(y)
