@@ -36,7 +36,7 @@ int tzh_linear_codes_launch(hipStream_t st, int num_cus, const void *x, int32_t 
                             const float *gamma, const float *beta, float eps, float *ln_ws, int64_t ln_ws_rows,
                             bool row_scale);
 
-bool tzh_linear_small_wins(int64_t m, int64_t k, int64_t n, bool f32, bool ln);
+bool tzh_linear_small_wins(int num_cus, int64_t m, int64_t k, int64_t n, bool f32, bool ln);
 int tzh_linear_small_launch(hipStream_t st, int num_cus, const void *x, int32_t x_dtype, const int8_t *q,
                             const uint16_t *scale, const float *bias, void *c, int32_t c_dtype, int64_t m, int64_t k,
                             int64_t n, int32_t epilogue, const void *res, float *pre_ln);
@@ -154,7 +154,7 @@ int linear(tzh_ctx *ctx, const void *a, int32_t a_dtype, const int8_t *wq, const
     if (((uintptr_t)c & 3) || (ln && !al16(c)))
         return tzh_fail(TZH_ERR_INVALID_ARGS, "c is not aligned to its element (16 bytes with the LayerNorm epilogue)");
     const Workspace wsz = workspace_of(ctx, a, a_dtype, m, k, n, ln);
-    if (tzh_linear_small_wins(m, k, n, a_dtype == TZH_F32, ln) && (!ln || m <= wsz.ws_rows)) {
+    if (tzh_linear_small_wins(ctx->num_cus, m, k, n, a_dtype == TZH_F32, ln) && (!ln || m <= wsz.ws_rows)) {
         // few rows: the codes and rows are read as they are, and the
         // LayerNorm epilogue's rows wait in the workspace
         float *rows = nullptr;

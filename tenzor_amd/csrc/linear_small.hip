@@ -499,21 +499,27 @@ int launch_small(hipStream_t st, int num_cus, const SmallArgs &a) {
 }  // namespace
 
 // Whether linear_small_kernel is the faster one for m rows: both times in us
-// as measured.  This kernel pays by the product (m n k in billions); the
-// pipelined one walks ceil(k / 64) serial stages once per 1536 columns
-// whatever m is, up to one round of tiles (beyond it this one has long
-// lost).  Measured, small / pipelined: f32 128 x 384 x 1152 5.2 / 27, 2048 x
+// as measured on an MI355X of 256 CUs.  This kernel pays by the product (m n k
+// in billions, over the CUs there are), nearly twice as much for f32 rows that
+// are not whole 16-byte pieces; the pipelined one walks ceil(k / 64) serial
+// stages once per 1536 columns whatever m is, up to one round of tiles (beyond
+// it this one has long lost), after passes over the rows and codes where k is
+// ragged.  Measured, small / pipelined: f32 128 x 384 x 1152 5.2 / 27, 2048 x
 // 384 x 1536 GELU 20.8 / 30.4, 4096 x 384 x 1536 35 / 33, LayerNorm k = 1536
-// with 1024 rows 25 / 74, 8192 rows 73 / 76, 197 x 1000 x 1537 10 / 119;
-// f16 128 x 384 x 1152 4.0 / 14.9, 2048 x 384 x 1536 11.7 / 18.5, 4096 rows
-// 22 / 19.6, LayerNorm k = 1536 with 1024 rows 17 / 21, 2048 rows 27 / 22.
-bool tzh_linear_small_wins(int64_t m, int64_t k, int64_t n, bool f32, bool ln) {
-    if (m > 16384) return false;
-    const double work = (double)m * (double)k * (double)n * 1e-9, stages = (double)((k + 63) / 64);
-    const double launches = (double)((n + 1535) / 1536);
-    if (f32) return (ln ? 8.0 : 4.0) + 14.0 * work < launches * (6.0 + 3.0 * stages);
-    if (!ln) return 3.0 + 7.5 * work < launches * (8.0 + 1.3 * stages);
-    return 8.0 + 16.0 * work < (k > 384 ? 20.0 : 8.0 + 1.3 * stages);
+// with 1000 rows 23 / 74, 6000 71 / 74, k = 384 with 4096 rows 21.8 / 27.6,
+// 6000 31.5 / 28.2; 197 x 1000 x 1537 11.5 / 119, 2048 x 2049 x 777 87 / 123,
+// 4096 x 2049 x 777 169 / 131; f16 128 x 384 x 1152 4.0 / 14.9, 2048 x 384 x
+// 1536 11.7 / 18.5, 4096 rows 22 / 19.6, LayerNorm k = 1536 with 1024 rows
+// 17 / 21, 2048 rows 27 / 22, k = 384 with 3000 rows 18.4 / 15.3.
+bool tzh_linear_small_wins(int num_cus, int64_t m, int64_t k, int64_t n, bool f32, bool ln) {
+    if (m > (int64_t)num_cus * 64) return false;
+    const double work = (double)m * (double)k * (double)n * 1e-9 * 256.0 / num_cus;
+    const double stages = (double)((k + 63) / 64), launches = (double)((n + 1535) / 1536);
+    const double pipe32 = launches * (6.0 + 3.0 * stages);
+    if (f32 && ln) return 8.0 + 14.0 * work < pipe32 && 12.0 + 18.0 * work < 10.5 + 2.75 * stages;
+    if (f32) return 4.0 + 14.0 * work < pipe32 && (k % 4 == 0 || 4.0 + 26.0 * work < pipe32 + 15.0);
+    if (!ln) return 3.5 + 7.5 * work < launches * (8.0 + 1.3 * stages);
+    return 8.5 + 18.0 * work < (k > 384 ? 20.0 : 8.0 + 1.3 * stages);
 }
 
 // C = epi(X q^T s + b) for caller-owned codes q [n, k] (row-major int8, any

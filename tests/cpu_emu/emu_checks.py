@@ -1012,7 +1012,35 @@ def group_launches():
             eval_launches(Tensor(Unbacked((b, m, k), dt)).matmul(Tensor(Unbacked((k, n), dt))))
 
 
-GROUPS = {"launches": group_launches, "eval": group_eval, "gemm_fp": group_gemm_fp, "gemm": group_gemm, "gemm_ln": group_gemm_ln, "range": group_range,
+def linear_kernel(m, k, n, dt, epi):
+    """The kernel that a caller-owned int8 linear's products run on."""
+    code, p = (_abi.F16 if dt == "f16" else _abi.F32), 1 << 40
+    names = [x[0] for x in launches_of(lambda: L.tzh_linear_w8(CTX, p, code, p, p, p, p, code, m, k, n, epi, p, code, p, p, 1e-12))]
+    kinds = {"small" for x in names if "linear_small_kernel" in x} | {"pipe" for x in names if "linear_pipe_kernel" in x}
+    assert len(kinds) == 1, names
+    return kinds.pop()
+
+
+def group_linear_rule():
+    """Which kernel a linear runs on, at sizes where both were timed (on 256
+    CUs) and one was at least a tenth faster; on fewer CUs the few-row kernel's
+    share of the work grows."""
+    B, G, N = _abi.EPI_BIAS, _abi.EPI_BIAS_GELU, _abi.EPI_BIAS_RES_LN
+    cus = int(os.environ.get("TZH_EMU_CUS", "16"))
+    small = [(128, 384, 1152, "f32", B), (2048, 384, 1536, "f32", G), (1000, 1536, 384, "f32", N), (4096, 384, 384, "f32", N),
+             (197, 1000, 1537, "f32", B), (2048, 2049, 777, "f32", B), (128, 384, 1152, "f16", B), (2048, 384, 1536, "f16", G),
+             (1000, 1536, 384, "f16", N)]
+    pipe = [(3000, 2049, 777, "f32", B), (4096, 1537, 777, "f32", B), (4096, 2049, 777, "f32", B), (6000, 384, 384, "f32", N),
+            (20000, 384, 384, "f32", B), (3000, 64, 384, "f16", N), (3000, 384, 384, "f16", N), (8192, 64, 1536, "f16", G)]
+    if cus == 256:
+        assert [linear_kernel(*c) for c in small] == ["small"] * len(small)
+        assert [linear_kernel(*c) for c in pipe] == ["pipe"] * len(pipe)
+    else:  # 16 CUs: a sixteenth of the rows
+        assert [linear_kernel((c[0] + 15) // 16, *c[1:]) for c in small] == ["small"] * len(small)
+        assert [linear_kernel(*c) for c in pipe + [(1000, 1536, 384, "f32", N), (2048, 384, 1536, "f16", G)]] == ["pipe"] * (len(pipe) + 2)
+
+
+GROUPS = {"launches": group_launches, "linear_rule": group_linear_rule, "linear_rule_256": group_linear_rule, "eval": group_eval, "gemm_fp": group_gemm_fp, "gemm": group_gemm, "gemm_ln": group_gemm_ln, "range": group_range,
           "attention": group_attention,
           "arctic": group_arctic, "arctic_f16w": group_arctic_f16w, "embed": group_embed, "models": group_models, "mlp": group_mlp,
           "mlp_split": group_mlp_split,

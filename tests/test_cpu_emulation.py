@@ -34,7 +34,7 @@ def emu_env():
     return env
 
 
-GROUPS = ["launches", "eval", "attention", "gemm", "gemm_ln", "range", "models", "nodes", "gemm_fp", "mlp", "mlp_split", "arctic",
+GROUPS = ["launches", "linear_rule", "linear_rule_256", "eval", "attention", "gemm", "gemm_ln", "range", "models", "nodes", "gemm_fp", "mlp", "mlp_split", "arctic",
           "arctic_f16w"]
 # emulated CU count per group (default 16): two CUs give the fused
 # feed-forward kernel blocks of several panels at a size the emulation
@@ -42,7 +42,8 @@ GROUPS = ["launches", "eval", "attention", "gemm", "gemm_ln", "range", "models",
 # one to three panels into 24, 12 and 8 parts; with four, the small
 # forwards of group arctic split their two panels in two, not eight (each
 # part repeats its panel's O-projection, which the emulation pays for)
-GROUP_ENV = {"mlp": {"TZH_EMU_CUS": "2"}, "mlp_split": {"TZH_EMU_CUS": "24"}, "arctic": {"TZH_EMU_CUS": "4"}}
+GROUP_ENV = {"linear_rule_256": {"TZH_EMU_CUS": "256"},
+             "mlp": {"TZH_EMU_CUS": "2"}, "mlp_split": {"TZH_EMU_CUS": "24"}, "arctic": {"TZH_EMU_CUS": "4"}}
 
 
 # test_gpu_eval.py's whole sequence in one process, in file order, with the
