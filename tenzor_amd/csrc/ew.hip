@@ -178,7 +178,8 @@ __global__ void __launch_bounds__(256) ew_chain_kernel(const EwProgram p, T *__r
 // Reductions of a chain over [outer, rsz, inner] along rsz: the bodies are
 // reduce_rows and reduce_cols of ew_shared.inc, here over one contiguous
 // leaf and over an interpreted program (contexts that ask for the
-// interpreter); other chains run them in generated kernels (ew_jit.cpp).
+// interpreter, and a program's first evaluation); other chains run them in
+// generated kernels (ew_jit.cpp).
 // Measured (kernel times, 16-byte loads, four vectors a thread, against one
 // thread a column or wave a row through the interpreter): mean over the
 // middle axis of f32 [256, 512, 384] 381 -> 37 us (5.4 TB/s); sum((x - y)^2)
@@ -1246,7 +1247,7 @@ struct Planner {
                 hipLaunchKernelGGL((ew_reduce_rows_kernel<T, V, LeafSrc<T, V>>), grid, dim3(256), 0, ctx->stream, src, a, dst);
             else
                 hipLaunchKernelGGL((ew_reduce_cols_kernel<T, V, LeafSrc<T, V>>), grid, dim3(256), 0, ctx->stream, src, a, dst);
-        } else if (kHaveJit && !ctx->ew_interpreter) {
+        } else if (kHaveJit && !ctx->ew_interpreter && jit_reduce_wanted(ctx, p, a, sizeof(T) == 8, V)) {
             TZH_TRY(jit_reduce_launch(ctx, p, a, sizeof(T) == 8, V, (int)blocks, dst));
         } else {
             const ProgSrc<T, V> src{p};

@@ -45,6 +45,9 @@ int jit_chain_launch(tzh_ctx *ctx, const EwProgram &p, bool f64, int V, int grid
 
 // The same for a reduction of program p: reduce_rows (a.inner == 1) or
 // reduce_cols over the generated operand, `grid` blocks of 256 threads.
+// jit_reduce_wanted: false where the interpreter should run it (a program's
+// first evaluation, and until it is compiled under stream capture).
+bool jit_reduce_wanted(tzh_ctx *ctx, const EwProgram &p, const RedArgs &a, bool f64, int V);
 int jit_reduce_launch(tzh_ctx *ctx, const EwProgram &p, const RedArgs &a, bool f64, int V, int grid, void *out);
 
 }  // namespace tzh_ew

@@ -308,6 +308,13 @@ hipError_t hipHostFree(void *p) { return hipFree(p); }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { std::memmove(d, s, n); return hipSuccess; }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(d, s, n, k); }
 hipError_t hipMemset(void *p, int v, size_t n) { std::memset(p, v, n); return hipSuccess; }
+// tzh_emu_capturing(1): streams answer that they are being captured
+static bool g_capturing = false;
+extern "C" void tzh_emu_capturing(int on) { g_capturing = on != 0; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *s) {
+    *s = g_capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipDeviceSynchronize() { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = new emu_stream; return hipSuccess; }

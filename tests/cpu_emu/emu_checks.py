@@ -1012,6 +1012,27 @@ def group_launches():
             eval_launches(Tensor(Unbacked((b, m, k), dt)).matmul(Tensor(Unbacked((k, n), dt))))
 
 
+def group_first_reductions():
+    """A chain's first reduction compiles nothing, nor does any under capture;
+    the second is generated; all give the same bits."""
+    rng = np.random.default_rng(40)
+    x = rng.standard_normal((9, 70)).astype(np.float32)
+    for axis in (1, 0):
+        e = lambda: ReduceExpr("sum", T(x).mul(0.5).tanh().sub(T(x)).exp(), (axis,))
+        generated = lambda: any("generated" in k for k, _, _ in eval_launches(e()))
+        L.tzh_emu_capturing(1)
+        assert not generated() and not generated(), axis  # (the second: not compiled yet, and not now)
+        L.tzh_emu_capturing(0)
+        assert generated(), axis
+        L.tzh_emu_capturing(1)
+        assert generated(), axis                          # (there already)
+        L.tzh_emu_capturing(0)
+        f = lambda: ReduceExpr("sum", T(x).abs().tanh().sub(T(x)).sub(0.25), (axis,))
+        first, second, third = (eval_both(f())[0] for _ in range(3))
+        assert np.array_equal(first, second) and np.array_equal(first, third), axis
+        assert any("generated" in k for k, _, _ in eval_launches(f()))
+
+
 def linear_kernel(m, k, n, dt, epi):
     """The kernel that a caller-owned int8 linear's products run on."""
     code, p = (_abi.F16 if dt == "f16" else _abi.F32), 1 << 40
@@ -1040,7 +1061,8 @@ def group_linear_rule():
         assert [linear_kernel(*c) for c in pipe + [(1000, 1536, 384, "f32", N), (2048, 384, 1536, "f16", G)]] == ["pipe"] * (len(pipe) + 2)
 
 
-GROUPS = {"launches": group_launches, "linear_rule": group_linear_rule, "linear_rule_256": group_linear_rule, "eval": group_eval, "gemm_fp": group_gemm_fp, "gemm": group_gemm, "gemm_ln": group_gemm_ln, "range": group_range,
+GROUPS = {"launches": group_launches, "first_reductions": group_first_reductions,
+          "linear_rule": group_linear_rule, "linear_rule_256": group_linear_rule, "eval": group_eval, "gemm_fp": group_gemm_fp, "gemm": group_gemm, "gemm_ln": group_gemm_ln, "range": group_range,
           "attention": group_attention,
           "arctic": group_arctic, "arctic_f16w": group_arctic_f16w, "embed": group_embed, "models": group_models, "mlp": group_mlp,
           "mlp_split": group_mlp_split,

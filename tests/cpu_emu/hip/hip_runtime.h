@@ -374,10 +374,7 @@ hipError_t hipMemset(void *p, int v, size_t n);
 hipError_t hipStreamSynchronize(hipStream_t s);
 hipError_t hipDeviceSynchronize();
 enum hipStreamCaptureStatus { hipStreamCaptureStatusNone, hipStreamCaptureStatusActive };
-inline hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *s) {
-    *s = hipStreamCaptureStatusNone;
-    return hipSuccess;
-}
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *s);
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned f);
 hipError_t hipStreamDestroy(hipStream_t s);
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned f);

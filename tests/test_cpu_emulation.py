@@ -34,8 +34,8 @@ def emu_env():
     return env
 
 
-GROUPS = ["launches", "linear_rule", "linear_rule_256", "eval", "attention", "gemm", "gemm_ln", "range", "models", "nodes", "gemm_fp", "mlp", "mlp_split", "arctic",
-          "arctic_f16w"]
+GROUPS = ["launches", "first_reductions", "linear_rule", "linear_rule_256", "eval", "attention", "gemm", "gemm_ln", "range",
+          "models", "nodes", "gemm_fp", "mlp", "mlp_split", "arctic", "arctic_f16w"]
 # emulated CU count per group (default 16): two CUs give the fused
 # feed-forward kernel blocks of several panels at a size the emulation
 # runs in about a minute (and a last round split in two); 24 CUs split

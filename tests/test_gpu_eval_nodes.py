@@ -10,7 +10,8 @@ import torch
 
 from oracle import eval_nodes as en
 
-from tenzor_amd.expr import LayerNormExpr, ReduceExpr, Tensor, eval
+import tenzor_amd
+from tenzor_amd.expr import LayerNormExpr, ReduceExpr, Tensor, eval, evalInto
 
 pytestmark = pytest.mark.gpu
 
@@ -104,6 +105,33 @@ def test_short_columns(dt, outer, n, inner):
     x[0, : n - 1, 0] = -np.inf
     tx = leaf(x)
     check_close(tx.softmax(1), {id(tx): x}, dt)
+
+
+def test_reduction_first_evaluated_under_capture():
+    """A chain's reduction whose first evaluation is captured (nothing is
+    compiled then), replayed over new inputs; later evaluations, by the
+    generated kernel, give the same bits."""
+    stream = torch.cuda.Stream()
+    x = torch.randn(33, 700, device="cuda")
+    out = torch.empty(33, device="cuda")
+    with torch.cuda.stream(stream):
+        c = tenzor_amd.Context(0)
+    expr = lambda: ReduceExpr("sum", Tensor(x).mul(0.5).sub(Tensor(x).abs()).mul(Tensor(x)).sub(0.125), (1,))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        evalInto(expr(), out, c)
+    for _ in range(3):
+        x.normal_()
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out.clone()
+        for _ in range(3):
+            evalInto(expr(), out, c)
+        torch.cuda.synchronize()
+        v = ((x * 0.5 - x.abs()) * x - 0.125).double()
+        assert torch.equal(out, got)
+        assert bool(((got.double() - v.sum(1)).abs() <= 2.0 ** -23 * 700 * v.abs().sum(1)).all())
 
 
 @pytest.mark.parametrize("perm", [(1, 0, 2, 3), (0, 2, 1, 3), (3, 2, 1, 0), (0, 1, 2, 3), (2, 0, 3, 1)])
