@@ -181,13 +181,18 @@ int tzh_eval_into(tzh_ctx *ctx, const tzh_node *tape, int32_t n_nodes,
  * whole f32 range: each row of a is scaled by an exact power of two 2^e
  * that puts its largest magnitude in [2^14, 2^15), each product a*q is
  * formed on the MFMA from an exact f16 split of the scaled value (hi + lo,
- * to 2^-22 relative for every value within 2^17 of its row's largest), the
+ * to 2^-22 relative for every value within 2^17 of its row's largest so far
+ * by 64 columns), the
  * sums run in f32 and are multiplied by 2^-e (exact) before the scale and
  * bias.  Rows holding inf or NaN give NaN where the reference gives inf or
  * NaN.  With few rows the codes are read where they are; otherwise they are
  * rewritten into the kernel's tiled format in the context scratch on every
  * call (with the row exponents, and a copy of a with zero columns when
- * k % 64 != 0). */
+ * k % 64 != 0).  The two kernels order their sums differently, so a row's last
+ * bits may differ between calls of few and of many rows (that of an f32 GEMM
+ * and of a reduction likewise between shapes, whose k or reduced axis may be
+ * split; a split also needs a workspace, so it may differ under stream
+ * capture). */
 int tzh_matmul_w8a32(tzh_ctx *ctx, const float *a, const int8_t *wq, const uint16_t *scale,
                      const float *bias, float *c, int64_t m, int64_t k, int64_t n);
 

@@ -1388,7 +1388,7 @@ struct Planner {
         else
             hipLaunchKernelGGL((ew_softmax_rows_kernel<T, V>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0,
                                ctx->stream, x, y, rows, len);
-        TZH_LAUNCHED("ew_softmax_rows_kernel");
+        TZH_LAUNCHED("softmax kernel over rows");
         return TZH_OK;
     }
 
@@ -1406,7 +1406,7 @@ struct Planner {
         else
             hipLaunchKernelGGL((ew_layernorm_kernel<T, V>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, ctx->stream,
                                x, g, b, y, rows, len, (T)1e-5f);
-        TZH_LAUNCHED("ew_layernorm_kernel");
+        TZH_LAUNCHED("LayerNorm kernel");
         return TZH_OK;
     }
 

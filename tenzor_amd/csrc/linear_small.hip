@@ -138,8 +138,9 @@ __global__ void __launch_bounds__(256, BM == 16 && WN == 4 && SCALED ? 3 : 2) li
 
     // A model's linears keep four partial sums, by the 64-code group modulo
     // four, added in order at the end: the same sums whether one wave holds
-    // all four or four waves one each, so a sequence's embedding does not
-    // depend on the tile, that is on the rest of its batch.
+    // all four or four waves one each, so among forwards on this kernel (up
+    // to tzh_small_layer_rows tokens) a sequence's embedding does not depend
+    // on the tile, that is on the rest of its batch.
     constexpr int NQ = WT ? 4 / WK : 1;
     f32x4_t acc[NQ][MF][NF];
 #pragma unroll

@@ -106,6 +106,35 @@ def test_hidden_states_layerwise(model, host, n_layers, dtype):
         off += L
 
 
+@pytest.mark.parametrize("n_layers", [1, 6])
+def test_hidden_states_of_the_fused_layers(model, host, n_layers):
+    """Layer by layer past 3.5 tokens a CU, where f32 layers run the fused
+    kernels."""
+    ids, lengths = synth.make_batch(22, 14, seq_len=96, min_len=64)
+    assert lengths.sum() > 3.5 * torch.cuda.get_device_properties(0).multi_processor_count
+    got = gpu_hidden(model, ids, lengths, n_layers)
+    start = np.concatenate([[0], np.cumsum(lengths)])
+    for b in (0, 6, 13):
+        err = np.abs(got[start[b]:start[b + 1]] - oracle.arctic_hidden(host, ids[b, :lengths[b]], n_layers))
+        assert err.max() < 1e-4 and np.sqrt((err ** 2).mean()) < 1e-5, (n_layers, b, float(err.max()))
+
+
+def test_embedding_bits_over_few_row_batches(model):
+    """A sequence's embedding is the same bits alone and in batches of about
+    400 and 850 tokens: 16 x 16, 16 x 64 and 32 x 64 tiles of the few-row
+    kernel, attention items in 1, 2 and 8 parts."""
+    rng = np.random.default_rng(23)
+    one = rng.integers(1000, 30522, 100).astype(np.uint32)
+    want = None
+    for others in ([], [150, 150], [150, 200, 130, 180, 90]):
+        lengths = np.array([100] + others, np.int32)
+        ids = rng.integers(1000, 30522, (len(lengths), lengths.max())).astype(np.uint32)
+        ids[0, :100] = one
+        got = gpu_embed(model, ids, lengths)[0]
+        want = got if want is None else want
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), lengths
+
+
 def test_f16_forward_within_north_star(model, host):
     """The opt-in f16 activation path still meets the north star's bar."""
     ids, lengths = synth.make_batch(24, 8, seq_len=256)

@@ -91,10 +91,28 @@ def test_matmul_w8a32_vs_oracle(ctx, m, k, n):
     assert (err <= bound(a, q, s, ref, k)).all(), float((err / bound(a, q, s, ref, k)).max())
 
 
-def test_matmul_w8a32_unaligned_operands(ctx):
+@pytest.mark.parametrize("m,k,n", [(16500, 385, 384), (17001, 130, 7), (16400, 1000, 1537), (20000, 40, 128)])
+def test_matmul_w8a32_ragged_past_the_few_rows(ctx, m, k, n):
+    """k tails, odd n and n over one 1536-column chunk on the pipelined
+    kernel: padded rows and codes (more rows than the few-row kernel is ever
+    used for), against float64 on sampled rows."""
+    a, q, s, bias = make_problem(m + n, m, k, n)
+    A, Q, S, B = dev(a), dev(q), dev(s.view(np.int16)), dev(bias)
+    Cg = torch.full((m, n), float("nan"), device="cuda")
+    check(lib().tzh_matmul_w8a32(ctx.handle, A.data_ptr(), Q.data_ptr(), S.data_ptr(), B.data_ptr(),
+                                 Cg.data_ptr(), m, k, n))
+    assert bool(torch.isfinite(Cg).all())
+    rows = np.unique(np.concatenate([np.arange(0, m, 97), np.arange(m - 130, m)]))
+    c = Cg.cpu().numpy()[rows]
+    lin = (a[rows].astype(np.float64) @ q.astype(np.float64).T) * s.view(np.float16).astype(np.float64) + bias
+    assert (np.abs(c - lin) <= bound(a[rows], q, s, lin, k)).all()
+
+
+@pytest.mark.parametrize("m,k,n", [(45, 130, 7), (16500, 130, 7), (16500, 128, 384)])
+def test_matmul_w8a32_unaligned_operands(ctx, m, k, n):
     """Row pitches that are not multiples of 16 bytes and operands that start
-    off 16-byte boundaries (views into larger buffers)."""
-    m, k, n = 45, 130, 7
+    off 16-byte boundaries (views into larger buffers), on the few-row and the
+    pipelined kernel."""
     a, q, s, bias = make_problem(17, m, k, n)
     Abuf = torch.zeros(m * k + 1, device="cuda")
     Abuf[1:] = dev(a).reshape(-1)

@@ -80,9 +80,10 @@ def test_split_rows_match_whole_tiles(ctx, extra_rows, k, dtype):
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
 def test_small_batch_is_all_pieces(ctx, dtype):
-    """Fewer tiles than CUs (config-1-like sizes): every tile is split
-    (k = 448), or the short-k configuration runs them (k = 384, f16)."""
-    for m, k in ((1, 448), (7, 448), (128, 384), (1000, 448), (1000, 384)):
+    """Fewer tiles than CUs: of a few thousand rows every tile is split
+    (k = 448), or the short-k configuration runs them (k = 384); fewer rows
+    run on the few-row kernel."""
+    for m, k in ((1, 448), (7, 448), (128, 384), (1000, 448), (1000, 384), (6001, 448), (6000, 384)):
         a, q, s, bias, res, g, b = problem(m, m, k, dtype)
         got = ln_gemm(ctx, a, q, s, bias, res, g, b)
         ref = oracle.layernorm(res.astype(np.float32) + oracle.matmul_w8a32(a.astype(np.float32), q, s, bias), g, b,

@@ -66,11 +66,29 @@ def inputs(seed, t):
 
 @pytest.mark.parametrize("t,layer", [(1, 0), (15, 1), (16, 0), (17, 1), (64, 0), (65, 1), (1000, 0), (4097, 1)])
 def test_fused_feed_forward_matches_oracle(model, weights, t, layer):
+    """Up to 2.5 rows a CU the linears one by one, then the fused kernel."""
     print(f"feed-forward t={t} layer={layer}", flush=True)
     x = inputs(t, t)
     got = gpu_ffn(model, layer, x).cpu().numpy()
     err = float(np.abs(got - ffn_oracle(weights, layer, x)).max())
     assert np.isfinite(got).all() and err < TOL, err
+
+
+@pytest.mark.parametrize("extra,layer", [(1, 0), (15, 1), (17, 0), (64, 1), (65, 0)])
+def test_fused_feed_forward_one_round_and_a_little(model, weights, extra, layer):
+    """A whole round of the fused kernel's 64-token panels, then one or two
+    panels split in as many parts as there are (24), against the oracle on
+    the split rows and a sample of the whole ones; the same rows by the few-row
+    kernel agree within the same bound."""
+    t = torch.cuda.get_device_properties(0).multi_processor_count * 64 + extra
+    print(f"feed-forward t={t} layer={layer}", flush=True)
+    x = inputs(extra, t)
+    got = gpu_ffn(model, layer, x).cpu().numpy()
+    rows = np.unique(np.concatenate([np.arange(t - extra - 3, t), np.arange(0, t, 997)]))
+    ref = ffn_oracle(weights, layer, x[rows])
+    assert np.isfinite(got).all() and float(np.abs(got[rows] - ref).max()) < TOL
+    few = gpu_ffn(model, layer, x[rows]).cpu().numpy()
+    assert float(np.abs(few - ref).max()) < TOL
 
 
 def test_fused_vs_gemm_pair_full_size(model, weights):
@@ -98,7 +116,7 @@ def test_rows_independent_of_placement(model, t):
     lane) among whole panels (16 384 tokens: 256 panels, one round) and
     among the parts of split ones (3001 tokens: all 47 panels split in four
     parts).  Whole and split panels add the chunks' sums in different
-    orders, so a token alone (split in 24 parts) is within the bound."""
+    orders, and a token alone runs the few-row kernel: within the bound."""
     print(f"feed-forward permutation t={t}", flush=True)
     x = torch.from_numpy(inputs(11, t)).cuda()
     perm = torch.from_numpy(np.random.default_rng(12).permutation(t)).cuda()
@@ -122,11 +140,15 @@ def test_feed_forward_edges(model):
         feedForward(y, x, model, CFG.num_hidden_layers, 32)
 
 
-def test_forward_with_and_without_fusion(model):
-    """The whole forward: embeddings with the fused block within 1e-5 of the
-    GEMM pair's (both f32 arithmetic)."""
+@pytest.mark.parametrize("batch,min_len", [(6, 3), (16, 100)])
+def test_forward_with_and_without_fusion(model, batch, min_len):
+    """The whole forward: embeddings within 1e-5 of the GEMM pair's (both f32
+    arithmetic), of a few hundred tokens (the few-row kernel) and of more than
+    3.5 a CU (the fused kernels)."""
     print("forward fused vs GEMM pair", flush=True)
-    ids, lengths = synth.make_batch(31, 6, seq_len=128, min_len=3)
+    ids, lengths = synth.make_batch(31, batch, seq_len=128, min_len=min_len)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert (lengths.sum() > 3.5 * cus) == (batch == 16)
     d_ids = torch.from_numpy(np.ascontiguousarray(ids).view(np.int32)).cuda()
     outs = []
     for fused in (True, False):

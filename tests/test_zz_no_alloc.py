@@ -41,8 +41,10 @@ def scratch_info(c):
     return nbytes.value, allocs.value
 
 
-@pytest.mark.parametrize("shapes", [[(2048, 1536, 384), (70, 384, 1152)],   # k % 64 == 0: codes only
-                                    [(1000, 385, 768), (33, 100, 5)]])       # k tails: padded rows too
+# the few-row kernel (no workspace), and past the rows it is ever used for
+# the pipelined one: k % 64 == 0, codes only, and k tails, padded rows too
+@pytest.mark.parametrize("shapes", [[(2048, 1536, 384), (70, 384, 1152)], [(1000, 385, 768), (33, 100, 5)],
+                                    [(20000, 448, 384), (17000, 384, 384)], [(17000, 385, 384), (16500, 100, 5)]])
 def test_noalloc_matches_allocating_entry(ctx, shapes):
     own = tenzor_amd.Context(0)  # runs the no-allocation entry point only
     try:
