@@ -496,7 +496,7 @@ __global__ void __launch_bounds__(256) ew_layernorm_held_kernel(const T *__restr
 // thread, so x is read once and y written once, in runs of 2^lx elements
 // (one thread a column passed over memory five times; transposing first and
 // after, six).  Measured, us: f32 [60000, 16, 64], one thread a column 250 ->
-// 121 (4.1 TB/s); through transposes f64 [1, 2000, 16] 38 -> 18, f32 [12, 13,
+// 86 (5.7 TB/s); through transposes f64 [1, 2000, 16] 38 -> 18, f32 [12, 13,
 // 217] 41 -> 8.6.
 template <typename T, int NP, int B>
 __global__ void __launch_bounds__(B) ew_softmax_cols_held_kernel(const T *__restrict__ x, T *__restrict__ y,

@@ -351,7 +351,8 @@ int emu_compile(const std::string &src, bool f64, bool reduce, EmuLaunch *out) {
     Dl_info info{};
     if (!dladdr((const void *)&jit_chain_launch, &info) || !info.dli_fname)
         return tzh_fail(TZH_ERR_DEVICE, "emulated chain kernel: cannot locate the emulation library");
-    const std::string stem = g_dir + "/k" + std::to_string(g_cache.size());
+    static int compiled = 0;  // (under g_mu)
+    const std::string stem = g_dir + "/k" + std::to_string(compiled++);
     const char *T = f64 ? "double" : "float";
     std::string text = "#include \"hip/hip_runtime.h\"\n" + src;
     const std::string kernel = reduce ? "tzh_reduce" : "tzh_chain";

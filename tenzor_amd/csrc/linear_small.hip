@@ -79,7 +79,7 @@ constexpr int kEUnset = 200;  // row exponent before any value: above every 15 -
 // BM rows by 16 NF WN outputs per block (NF fragments of 16 a wave), 4 / WN
 // waves over each chunk's k.
 template <typename TX, typename TC, typename TR, int EPI, bool WT, bool SCALED, bool LNP, int BM, int WN, int NF>
-__global__ void __launch_bounds__(256, BM == 16 && WN == 4 && SCALED ? 3 : 2) linear_small_kernel(const SmallArgs a) {
+__global__ void __launch_bounds__(256, !SCALED ? 1 : BM == 16 && WN == 4 ? 3 : 2) linear_small_kernel(const SmallArgs a) {
     constexpr bool SPLIT = sizeof(TX) == 4;
     constexpr int WK = 4 / WN, KC = WK == 1 ? 512 : 1024, P = KC + 8, MF = BM / 16;
     constexpr int TPR = 256 / BM;             // threads per row
@@ -201,7 +201,7 @@ __global__ void __launch_bounds__(256, BM == 16 && WN == 4 && SCALED ? 3 : 2) li
         for (int i = 0; i < NP; i++)
             if (8 * TPR * i < 64 * groups) {
                 const int j = c0 + 8 * (tl % TPR + TPR * i);
-                if (c0 + 8 * TPR * (i + 1) <= a.k) {
+                if (WT || c0 + 8 * TPR * (i + 1) <= a.k) {  // (a model's k: whole pieces)
                     __builtin_memcpy(xv[i], row + j, 8 * sizeof(TX));  // (16-byte loads; element alignment is enough)
                 } else {  // the row's last piece: what lies past it is cleared where it is used
 #pragma unroll
@@ -221,7 +221,7 @@ __global__ void __launch_bounds__(256, BM == 16 && WN == 4 && SCALED ? 3 : 2) li
         const int groups = groups_of(c0);
 #pragma unroll
         for (int i = 0; i < NP; i++)
-            if (8 * TPR * i < 64 * groups && c0 + 8 * TPR * (i + 1) > a.k)
+            if (!WT && 8 * TPR * i < 64 * groups && c0 + 8 * TPR * (i + 1) > a.k)
 #pragma unroll
                 for (int e = 0; e < 8; e++)
                     if (c0 + 8 * (sub + TPR * i) + e >= a.k) xv[i][e] = (TX)0;
@@ -562,7 +562,7 @@ int64_t tzh_small_layer_rows(int num_cus) { return (int64_t)num_cus * 7 / 2; }
 int64_t tzh_small_ffn_rows(int num_cus) { return (int64_t)num_cus * 5 / 2; }
 
 // A model linear over f32 rows inside the split's range (not row-scaled):
-// C = epi(X W^T s + b) with W8T codes, n a multiple of 384 and k of 64, all
+// C = epi(X W^T s + b) with W8T codes, n a multiple of 384 and k of 128, all
 // pointers 16-byte aligned.  epilogue: TZH_EPI_BIAS, TZH_EPI_BIAS_GELU, or
 // TZH_EPI_BIAS_RES_LN for the rows before the LayerNorm (res added).  gamma
 // non-null (k == 384): x holds rows before a LayerNorm, normalised on the
@@ -570,7 +570,7 @@ int64_t tzh_small_ffn_rows(int num_cus) { return (int64_t)num_cus * 5 / 2; }
 int tzh_linear_small_model_launch(hipStream_t st, int num_cus, const float *x, const float *gamma, const float *beta,
                                   float eps, float *xout, const void *w, const uint16_t *scale, const float *bias,
                                   float *c, int64_t m, int64_t k, int64_t n, int32_t epilogue, const float *res) {
-    if (m <= 0 || m > ((int64_t)1 << 20) || k % 64 || n % 384 || (gamma && (k != 384 || !beta || !xout)))
+    if (m <= 0 || m > ((int64_t)1 << 20) || k % 128 || n % 384 || (gamma && (k != 384 || !beta || !xout)))
         return tzh_fail(TZH_ERR_INVALID_ARGS, "internal: bad small linear");
     SmallArgs a{};
     a.x = x, a.w = w, a.scale = scale, a.bias = bias, a.c = c, a.res = res;
